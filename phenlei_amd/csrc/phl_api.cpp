@@ -372,29 +372,30 @@ phl_status check_sweep_waits(phl_ctx *c)
     return PHL_OK;
 }
 
-// Real cells of one cell-indexed row from storage order to mesh order (in place).
-void row_to_mesh(const phl_ctx *c, double *row, std::vector<double> &tmp)
+// Device rows of rowLen cell-indexed values (storage order) into host rows of
+// outRowLen values in mesh order (zero padded).  The rows are put in mesh
+// order on the device, in the update target qAlt (at least 5 nTotal values,
+// dead between calls), and leave in one copy.
+template <typename T>
+phl_status copy_field_t(phl_ctx *c, const T *dsrc, int rows, int rowLen, int outRowLen, double *out)
 {
-    const int nC = (int)c->cellAt.size();
-    tmp.assign(row, row + nC);
-    for (int i = 0; i < nC; ++i) row[c->cellAt[i]] = tmp[i];
+    if (rows > 5 || outRowLen > c->m.nTotal) return fail(PHL_ERR_ARG, "field rows exceed the staging array");
+    phl::launch_cells_out(c->m, dsrc, rows, rowLen, outRowLen, c->f.qAlt, c->stream);
+    HIPTRY(hipGetLastError());
+    HIPTRY(hipMemcpyAsync(out, c->f.qAlt, sizeof(double) * (size_t)rows * outRowLen, hipMemcpyDeviceToHost, c->stream));
+    HIPTRY(hipStreamSynchronize(c->stream));
+    return PHL_OK;
 }
 
 phl_status copy_field(phl_ctx *c, const double *dsrc, int rows, int rowLen, int outRowLen, double *out)
 {
-    // rows of rowLen device values (cell-indexed, storage order) into rows of
-    // outRowLen host values in mesh order (zero padded)
-    for (int r = 0; r < rows; ++r) {
-        double *o = out + (size_t)r * outRowLen;
-        if (rowLen > 0)
-            HIPTRY(hipMemcpyAsync(o, dsrc + (size_t)r * rowLen, (size_t)rowLen * sizeof(double),
-                                  hipMemcpyDeviceToHost, c->stream));
-        for (int i = rowLen; i < outRowLen; ++i) o[i] = 0.0;
-    }
-    HIPTRY(hipStreamSynchronize(c->stream));
-    std::vector<double> tmp;
-    for (int r = 0; r < rows && rowLen >= c->m.nCell; ++r) row_to_mesh(c, out + (size_t)r * outRowLen, tmp);
-    return PHL_OK;
+    return copy_field_t(c, dsrc, rows, rowLen, outRowLen, out);
+}
+
+// FP32 rows (mixed-form gradients), widened to FP64 on the way.
+phl_status copy_field_f32(phl_ctx *c, const float *dsrc, int rows, int rowLen, int outRowLen, double *out)
+{
+    return copy_field_t(c, dsrc, rows, rowLen, outRowLen, out);
 }
 
 // The five components of a [n][kRow] device array (n rows, storage order)
@@ -405,42 +406,23 @@ phl_status copy_rows(phl_ctx *c, const double *dsrc, int n, int outRowLen, doubl
     if (n > 0)
         HIPTRY(hipMemcpyAsync(h.data(), dsrc, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
     HIPTRY(hipStreamSynchronize(c->stream));
+    const int nC = c->m.nCell;
     for (int m = 0; m < 5; ++m) {
         double *o = out + (size_t)m * outRowLen;
-        for (int i = 0; i < outRowLen; ++i) o[i] = i < n ? h[(size_t)i * phl::kRow + m] : 0.0;
+        for (int i = 0; i < outRowLen; ++i)
+            o[i] = i < n ? h[(size_t)(i < nC ? c->slotOf[i] : i) * phl::kRow + m] : 0.0;
     }
-    std::vector<double> tmp;
-    for (int m = 0; m < 5 && n >= c->m.nCell; ++m) row_to_mesh(c, out + (size_t)m * outRowLen, tmp);
     return PHL_OK;
 }
 
-// Host rows of rowLen cell-indexed values (mesh order) to the device (storage order).
+// Host rows of rowLen cell-indexed values (mesh order) to the device (storage
+// order), staged in qAlt as the reads are.
 phl_status upload_cells(phl_ctx *c, double *ddst, int rows, int rowLen, const double *in)
 {
-    const int nC = c->m.nCell;
-    std::vector<double> h(in, in + (size_t)rows * rowLen);
-    for (int r = 0; r < rows; ++r) {
-        double *o = h.data() + (size_t)r * rowLen;
-        const double *src = in + (size_t)r * rowLen;
-        for (int i = 0; i < nC && i < rowLen; ++i) o[c->slotOf[i]] = src[i];
-    }
-    HIPTRY(hipMemcpyAsync(ddst, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, c->stream));
+    HIPTRY(hipMemcpyAsync(c->f.qAlt, in, sizeof(double) * (size_t)rows * rowLen, hipMemcpyHostToDevice, c->stream));
+    phl::launch_cells_in(c->m, c->f.qAlt, rows, rowLen, ddst, c->stream);
+    HIPTRY(hipGetLastError());
     HIPTRY(hipStreamSynchronize(c->stream));
-    return PHL_OK;
-}
-
-// FP32 rows (mixed-form gradients) widened to FP64 on the host.
-phl_status copy_field_f32(phl_ctx *c, const float *dsrc, int rows, int rowLen, int outRowLen, double *out)
-{
-    std::vector<float> tmp((size_t)rows * rowLen);
-    if (!tmp.empty())
-        HIPTRY(hipMemcpyAsync(tmp.data(), dsrc, tmp.size() * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    HIPTRY(hipStreamSynchronize(c->stream));
-    for (int r = 0; r < rows; ++r)
-        for (int i = 0; i < outRowLen; ++i)
-            out[(size_t)r * outRowLen + i] = i < rowLen ? (double)tmp[(size_t)r * rowLen + i] : 0.0;
-    std::vector<double> t2;
-    for (int r = 0; r < rows && rowLen >= c->m.nCell; ++r) row_to_mesh(c, out + (size_t)r * outRowLen, t2);
     return PHL_OK;
 }
 

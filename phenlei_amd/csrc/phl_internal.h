@@ -255,6 +255,13 @@ struct Levels {
 };
 
 // Launchers (phl_kernels.hip).  All are asynchronous on `s`.
+// Cell-indexed rows between the device's storage order and the mesh's order:
+// out, [rows][rowLen] -> [rows][outLen] zero padded; in, [rows][rowLen].
+void launch_cells_out(const DevMesh &m, const double *src, int rows, int rowLen, int outLen, double *dst,
+                      hipStream_t s);
+void launch_cells_out(const DevMesh &m, const float *src, int rows, int rowLen, int outLen, double *dst,
+                      hipStream_t s);
+void launch_cells_in(const DevMesh &m, const double *src, int rows, int rowLen, double *dst, hipStream_t s);
 void launch_boundary(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s);
 void launch_gamma_t(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s);
 // The gradients go to the gather records (the face loop and the SA source

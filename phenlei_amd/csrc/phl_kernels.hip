@@ -2497,6 +2497,32 @@ __global__ void __launch_bounds__(1024) k_fix(DevMesh M, Consts K0, const double
 
 inline int nblk(int n, int b) { return (n + b - 1) / b; }
 
+// Cell-indexed rows from storage order to mesh order (out; widened to FP64,
+// zero padded) and back (in), one thread per cell of the destination, whose
+// accesses are coalesced; ghosts keep their index.  The source side is a
+// gather of 8-byte values, about a tenth of the host transfer it stands next
+// to: with the permutation on one host core, reading a 1.01M-cell state took
+// 6.2 ms and loading one 7.4 ms.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_cells_out(DevMesh M, const T *__restrict__ src, int rows, int rowLen,
+                                                      int outLen, double *__restrict__ dst)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= outLen) return;
+    const int j = i < M.nCell ? M.cellAt[i] : i;
+    for (int r = 0; r < rows; ++r)
+        dst[(size_t)r * outLen + i] = i < rowLen ? double(src[(size_t)r * rowLen + j]) : 0.0;
+}
+
+__global__ void __launch_bounds__(kBlock) k_cells_in(DevMesh M, const double *__restrict__ src, int rows, int rowLen,
+                                                     double *__restrict__ dst)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= rowLen) return;
+    const int j = i < M.nCell ? M.logicalOf[i] : i;
+    for (int r = 0; r < rows; ++r) dst[(size_t)r * rowLen + i] = src[(size_t)r * rowLen + j];
+}
+
 // Streaming copy used to measure achievable HBM bandwidth.
 __global__ void __launch_bounds__(kBlock) k_copy(const double2 *__restrict__ src, double2 *__restrict__ dst,
                                                  size_t n)
@@ -2609,6 +2635,25 @@ void launch_copy(const double *src, double *dst, size_t n, hipStream_t s)
 }
 
 // ------------------------------------------------------------ launchers
+void launch_cells_out(const DevMesh &m, const double *src, int rows, int rowLen, int outLen, double *dst,
+                      hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cells_out<double>, dim3(nblk(outLen, kBlock)), dim3(kBlock), 0, s, m, src, rows, rowLen,
+                       outLen, dst);
+}
+
+void launch_cells_out(const DevMesh &m, const float *src, int rows, int rowLen, int outLen, double *dst,
+                      hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cells_out<float>, dim3(nblk(outLen, kBlock)), dim3(kBlock), 0, s, m, src, rows, rowLen,
+                       outLen, dst);
+}
+
+void launch_cells_in(const DevMesh &m, const double *src, int rows, int rowLen, double *dst, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cells_in, dim3(nblk(rowLen, kBlock)), dim3(kBlock), 0, s, m, src, rows, rowLen, dst);
+}
+
 void launch_boundary(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s)
 {
     if (m.nBFace == 0) return;
