@@ -69,10 +69,10 @@ typedef struct phl_params {
     int cfl_vary_step;      /* CFLVaryStep (500) */
     int n_lusgs_sweeps;     /* nLUSGSSweeps (1) */
     int precision;          /* 0 FP64; 1 mixed (FP32 gradients and face fluxes, FP64 accumulation/LU-SGS) */
-    int storage_order;      /* device storage of the cells: 0 locality order (cells sorted along a
-                             * Morton curve of their centroids, per case; default), 1 the mesh's order.
-                             * Results do not depend on it: every sweep and accumulation follows the
-                             * mesh's cell and face numbering either way. */
+    int storage_order;      /* device storage of the cells: 0 (default) by LU-SGS level and, within a
+                             * level, by the storage positions of the swept neighbours, per case; 1 the
+                             * mesh's order.  Results do not depend on it: every sweep and accumulation
+                             * follows the mesh's cell and face numbering either way. */
     int face_loop;          /* 0 (default): face kernel + cell gather, face values through HBM; 1:
                              * tile-fused (a workgroup evaluates the faces of its cells into LDS and sums
                              * them; faces between tiles are evaluated twice).  Identical results; the

@@ -1,8 +1,8 @@
 // phl_internal.h -- device data layout shared by the kernels and the host
 // driver.  Not part of the C-ABI.
 //
-// Cell-indexed arrays are in storage order (a locality order of the real
-// cells, then the ghosts of boundary faces 0..nBFace-1); faces keep the
+// Cell-indexed arrays are in storage order (an order of the real cells that
+// follows the sweep levels, then the ghosts of boundary faces 0..nBFace-1); faces keep the
 // mesh's numbering.
 //
 // Layout in HBM (FP64 plain form):
@@ -58,7 +58,7 @@ struct DevMesh {
     const unsigned short *caseOf;  // [nTotal] case of each cell (batched contexts)
     const int *caseCellPtr;        // [nCases+1] cell range of each case
     const double *wallDist;        // [nCell] distance to the nearest solid surface (SA)
-    // Cells are stored in a locality order; the sweeps and SolutionFix follow
+    // Cells are stored in the order of the sweep levels; sweeps and SolutionFix follow
     // the mesh's own numbering through these maps (ghost cells are not moved).
     const int *logicalOf;          // [nCell] mesh index of the cell stored at each position
     const int *cellAt;             // [nCell] storage position of each mesh cell
