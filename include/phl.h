@@ -80,8 +80,8 @@ typedef struct phl_params {
                              * 0.39 vs 0.32 ms). */
     int sweep_form;         /* LU-SGS sweeps (identical results: same arithmetic and summation order):
                              * 0 (default) dataflow, one launch per direction: chunks of 64 cells of
-                             * the level order, each wavefront waiting on the flags of the chunks that
-                             * hold its cells' swept neighbours, chunks taken in launch order;
+                             * the level order, each wavefront polling its swept neighbours' increments
+                             * until they are there, chunks taken in launch order;
                              * 1 one launch per dependency level;
                              * 2 dataflow with chunks taken from a ticket counter (independent of the
                              * workgroup dispatch order; slower on large meshes);

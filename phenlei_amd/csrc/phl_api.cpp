@@ -65,6 +65,7 @@ struct phl_ctx {
     // saDeferred: a relaxation is waiting for its sweeps and update.
     bool saFused = false;
     bool saDeferred = false;
+    bool sweepGaveUp = false;  // a dataflow sweep exceeded its wait bound since the last new state
     // phl_solve / phl_solve_batch: switch a mixed context to FP64 once no
     // unconverged case has halved its residual for this many steps (0: never)
     int precisionSwitchStall = 0;
@@ -204,46 +205,54 @@ void build_sweep_order(int nC, const std::vector<int> &c2fPtr, const std::vector
 
 // The dataflow sweep's order (phl::FlowOrder) for one direction: each level
 // of `cells` (mesh numbers, level order) padded to whole chunks of 64
-// positions, the slot lists of build_sweep_order moved along (row, nb in mesh
-// numbers; converted to storage here), and per chunk the distinct chunks
-// holding its real neighbours, all of earlier levels.
+// positions, and the slot lists of build_sweep_order moved along (row, nb in
+// mesh numbers; converted to storage here), the boundary faces, which come
+// first in every list, apart from the real neighbours.
 phl_status build_flow_order(phl_ctx *c, int nC, const std::vector<int> &cells, const std::vector<int> &lptr,
                             const std::vector<int> &row, const std::vector<int> &nb, int Wa,
                             const std::vector<int> &slotOf, phl::FlowOrder &fo)
 {
-    int nCh = 0;
+    int nCh = 0, W = 0, WG = 0;
     for (size_t L = 0; L + 1 < lptr.size(); ++L) nCh += (lptr[L + 1] - lptr[L] + 63) / 64;
+    for (int pos = 0; pos < nC; ++pos) {
+        int g = 0, n = 0;
+        for (int s = 0; s < Wa && row[(size_t)s * nC + pos] >= 0; ++s) ++(nb[(size_t)s * nC + pos] >= nC ? g : n);
+        W = std::max(W, n);
+        WG = std::max(WG, g);
+    }
+    W = W <= 3 ? 3 : (W <= 4 ? 4 : 6);
     const size_t Pp = (size_t)64 * nCh;
-    std::vector<int> fc(Pp, -1), frow((size_t)Wa * Pp, -1), fnb((size_t)Wa * Pp, 0), chunkOf(nC, -1);
-    std::vector<int> depPtr(1, 0), dep, d;
+    std::vector<int> fc(Pp, -1), frow((size_t)W * Pp, -1), fnb((size_t)W * Pp, 0), frowG((size_t)WG * Pp, -1);
+    std::vector<int> chunkOf(nC, -1), width(std::max(nCh, 1), 0), widthG(std::max(nCh, 1), 0);
     int ch = 0;
     for (size_t L = 0; L + 1 < lptr.size(); ++L) {
         const int levelChunk0 = ch;
         for (int b = lptr[L]; b < lptr[L + 1]; b += 64, ++ch) {
-            d.clear();
             for (int j = 0; j < 64 && b + j < lptr[L + 1]; ++j) {
                 const int pos = b + j;
                 const size_t q = (size_t)ch * 64 + j;
                 fc[q] = slotOf[cells[pos]];
                 chunkOf[cells[pos]] = ch;
+                int g = 0, n = 0;
                 for (int s = 0; s < Wa; ++s) {
-                    const int r = row[(size_t)s * nC + pos], n = nb[(size_t)s * nC + pos];
-                    frow[(size_t)s * Pp + q] = r;
-                    fnb[(size_t)s * Pp + q] = n < nC ? slotOf[n] : n;
-                    if (r < 0 || n >= nC) continue;
+                    const int r = row[(size_t)s * nC + pos], o = nb[(size_t)s * nC + pos];
+                    if (r < 0) break;
+                    if (o >= nC) {
+                        if (n > 0) return fail(PHL_ERR_ARG, "dataflow sweep order: a boundary face follows an interior one");
+                        frowG[(size_t)g++ * Pp + q] = r;
+                        continue;
+                    }
                     // a neighbour swept earlier lies in a chunk of an earlier level
-                    if (chunkOf[n] < 0 || chunkOf[n] >= levelChunk0)
+                    if (chunkOf[o] < 0 || chunkOf[o] >= levelChunk0)
                         return fail(PHL_ERR_ARG, "dataflow sweep order: a neighbour is not in an earlier level");
-                    d.push_back(chunkOf[n]);
+                    frow[(size_t)n * Pp + q] = r;
+                    fnb[(size_t)n++ * Pp + q] = slotOf[o];
                 }
+                width[ch] = std::max(width[ch], n);
+                widthG[ch] = std::max(widthG[ch], g);
             }
-            std::sort(d.begin(), d.end());
-            d.erase(std::unique(d.begin(), d.end()), d.end());
-            dep.insert(dep.end(), d.begin(), d.end());
-            depPtr.push_back((int)dep.size());
         }
     }
-    if (dep.empty()) dep.push_back(0);  // keeps the device pointer valid
     // XCD groups (sweep_form 3): block ids rise with the level, as in launch
     // order, so the in-order dispatch argument for progress is unchanged; the
     // padding blocks of a level return at once
@@ -258,20 +267,19 @@ phl_status build_flow_order(phl_ctx *c, int nC, const std::vector<int> &cells, c
         }
         if (blockChunk.empty()) blockChunk.push_back(-1);
     }
-    std::vector<int> width(std::max(nCh, 1), 0);
-    for (int k = 0; k < nCh; ++k)
-        for (int j = 0; j < 64; ++j)
-            for (int s = 0; s < Wa; ++s)
-                if (frow[(size_t)s * Pp + (size_t)k * 64 + j] >= 0) width[k] = std::max(width[k], s + 1);
     const int *t;
     TRY(upload(c, &t, width)); fo.width = t;
     TRY(upload(c, &t, fc)); fo.cells = t;
     TRY(upload(c, &t, frow)); fo.row = t;
     TRY(upload(c, &t, fnb)); fo.nb = t;
-    TRY(upload(c, &t, depPtr)); fo.depPtr = t;
-    TRY(upload(c, &t, dep)); fo.dep = t;
+    TRY(upload(c, &t, widthG)); fo.widthG = t;
+    fo.rowG = nullptr;
+    if (WG > 0) {
+        TRY(upload(c, &t, frowG)); fo.rowG = t;
+    }
     TRY(upload(c, &t, blockChunk)); fo.blockChunk = t;
     fo.nBlocks = (int)blockChunk.size();
+    fo.W = W;
     fo.nChunks = nCh;
     return PHL_OK;
 }
@@ -366,9 +374,11 @@ phl_status check_sweep_waits(phl_ctx *c)
     int gaveUp = 0;
     HIPTRY(hipMemcpyAsync(&gaveUp, c->f.sweepCtl + 2, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPTRY(hipStreamSynchronize(c->stream));
-    if (gaveUp != 0)
+    if (gaveUp != 0) {
+        c->sweepGaveUp = true;
         return fail(PHL_ERR_NUMERIC, "dataflow sweep: " + std::to_string(gaveUp) +
                                          " wavefronts exceeded the wait bound; the state is invalid");
+    }
     return PHL_OK;
 }
 
@@ -398,19 +408,20 @@ phl_status copy_field_f32(phl_ctx *c, const float *dsrc, int rows, int rowLen, i
     return copy_field_t(c, dsrc, rows, rowLen, outRowLen, out);
 }
 
-// The five components of a [n][kRow] device array (n rows, storage order)
-// into five host rows of outRowLen values in mesh order (zero padded).
+// The five components of a device array of n rows in pair planes (storage
+// order) into five host rows of outRowLen values in mesh order (zero padded).
 phl_status copy_rows(phl_ctx *c, const double *dsrc, int n, int outRowLen, double *out)
 {
-    std::vector<double> h((size_t)phl::kRow * n);
+    const size_t N = (size_t)n;
+    std::vector<double> h(2 * phl::kPlanes * N);
     if (n > 0)
         HIPTRY(hipMemcpyAsync(h.data(), dsrc, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
     HIPTRY(hipStreamSynchronize(c->stream));
     const int nC = c->m.nCell;
     for (int m = 0; m < 5; ++m) {
         double *o = out + (size_t)m * outRowLen;
-        for (int i = 0; i < outRowLen; ++i)
-            o[i] = i < n ? h[(size_t)(i < nC ? c->slotOf[i] : i) * phl::kRow + m] : 0.0;
+        const double *src = h.data() + (m / 2) * 2 * N + m % 2;
+        for (int i = 0; i < outRowLen; ++i) o[i] = i < n ? src[2 * (size_t)(i < nC ? c->slotOf[i] : i)] : 0.0;
     }
     return PHL_OK;
 }
@@ -1183,9 +1194,9 @@ static phl_status create_impl(phl_ctx *c, const phl::Mesh &m)
         std::vector<int> row, nbs;
         build_sweep_order(nC, c2fPtr, c2fS, c2n, isLeft, dir == 0 ? cellsF : cellsB, dir == 0, lv.so.W, lv.so.Wpad,
                           row, nbs);
-        // the dataflow sweep addresses dq rows through a buffer descriptor
-        // with a 32-bit byte range; larger meshes take the level form
-        const bool rowsAddressable = (size_t)m.nTotal() * phl::kRow * sizeof(double) <= (size_t)INT32_MAX;
+        // the dataflow sweep addresses dq through a buffer descriptor with a
+        // 32-bit byte range; larger meshes take the level form
+        const bool rowsAddressable = (size_t)m.nTotal() * 2 * phl::kPlanes * sizeof(double) <= (size_t)INT32_MAX;
         if (p.sweep_form != 1 && lv.so.Wpad <= 6 && rowsAddressable)
             TRY(build_flow_order(c, nC, dir == 0 ? cellsF : cellsB, dir == 0 ? c->hfwdPtr : c->hbwdPtr, row, nbs,
                                  lv.so.Wpad, slotOf, lv.flow));
@@ -1276,8 +1287,14 @@ static phl_status create_impl(phl_ctx *c, const phl::Mesh &m)
         HIPTRY(hipMemset(fl.rtem, 0, sizeof(double) * nT));
     }
     k.rtem = fl.rtem;
-    TRY(dalloc(c, &fl.dq, (size_t)phl::kRow * nT));
-    TRY(dalloc(c, &fl.dflux, (size_t)phl::kRow * nC));
+    TRY(dalloc(c, &fl.dq, (size_t)2 * phl::kPlanes * nT));
+    TRY(dalloc(c, &fl.dflux, (size_t)2 * phl::kPlanes * nC));
+    fl.dqAlt = nullptr;
+    fl.bwdFlow = c->bwd.flow.nChunks > 0;
+    if (c->fwd.flow.nChunks > 0 || fl.bwdFlow) {
+        TRY(dalloc(c, &fl.dqAlt, (size_t)2 * phl::kPlanes * nT));
+        phl::launch_mark_dq(dm, fl.dqAlt, c->stream);
+    }
     TRY(dalloc(c, &fl.specInv, (size_t)nC));
     TRY(dalloc(c, &fl.specVis, (size_t)nC));
     TRY(dalloc(c, &fl.dtLoc, (size_t)nC));
@@ -1301,9 +1318,6 @@ static phl_status create_impl(phl_ctx *c, const phl::Mesh &m)
     // LU-SGS face coefficients, stored only for the level form (the dataflow
     // sweeps evaluate them)
     TRY(dalloc(c, &fl.coef, k.coefInSweep ? (size_t)16 : (size_t)nF * 2 * 16));
-    const int nChunks = std::max({c->fwd.flow.nChunks, c->bwd.flow.nChunks, 1});
-    TRY(dalloc(c, &fl.sweepFlag, (size_t)nChunks));
-    HIPTRY(hipMemset(fl.sweepFlag, 0, sizeof(int) * nChunks));
     TRY(dalloc(c, &fl.casePart, (size_t)nCases * 32 * 6));
     TRY(dalloc(c, &fl.sweepCtl, 4));
     {
@@ -1398,8 +1412,8 @@ static phl_status create_impl(phl_ctx *c, const phl::Mesh &m)
     HIPTRY(hipMemset(fl.res, 0, sizeof(double) * 5 * nC));
     HIPTRY(hipMemset(fl.grad, 0, sizeof(double) * 15 * nC));
     HIPTRY(hipMemset(fl.gradT, 0, sizeof(double) * 3 * nC));
-    HIPTRY(hipMemset(fl.dq, 0, sizeof(double) * phl::kRow * nT));
-    HIPTRY(hipMemset(fl.dflux, 0, sizeof(double) * phl::kRow * nC));
+    HIPTRY(hipMemset(fl.dq, 0, sizeof(double) * 2 * phl::kPlanes * nT));
+    HIPTRY(hipMemset(fl.dflux, 0, sizeof(double) * 2 * phl::kPlanes * nC));
     HIPTRY(hipMemset(fl.specVis, 0, sizeof(double) * nC));
     HIPTRY(hipMemset(fl.negFlag, 0, (size_t)nC));
     HIPTRY(hipMemset(fl.negCount, 0, sizeof(int)));
@@ -1486,8 +1500,12 @@ phl_status phl_create_batch(const phl_mesh *pm, const phl_params *params, int de
 // ---------------------------------------------------------------- state
 // A new state makes the context valid again after a sweep gave up waiting:
 // the count of waves that gave up is cleared with the state.
+// A new state: no sweep has given up on it.  Sweeps that did left rows of the
+// next sweep's buffer unmarked.
 static phl_status clear_gave_up(phl_ctx *c)
 {
+    if (c->sweepGaveUp && c->f.dqAlt) phl::launch_mark_dq(c->m, c->f.dqAlt, c->stream);
+    c->sweepGaveUp = false;
     HIPTRY(hipMemsetAsync(c->f.sweepCtl + 2, 0, sizeof(int), c->stream));
     HIPTRY(hipStreamSynchronize(c->stream));
     return PHL_OK;
@@ -1789,8 +1807,10 @@ phl_status phl_time_step(phl_ctx *c, int step)
     return check_launch(c);
 }
 
-// Controller::LUSGS with nLUSGSSweeps > 1 (Controller.cpp:1878-1961): dq
-// and LUplusDQ start from zero; after every sweep pair the squared change of
+// Controller::LUSGS with nLUSGSSweeps > 1 (Controller.cpp:1878-1961): LUplusDQ
+// starts from zero, and so does the dq that the first change is taken from (a
+// sweep reads only increments that it or the ghost kernel has just
+// written); after every sweep pair the squared change of
 // dq over both half-sweeps (the reference's sweepNormal, summed here in block
 // order) is read back, and the pairs stop once it falls below
 // LUSGSTolerance times the first pair's.  The host decides, so such steps
@@ -1799,17 +1819,16 @@ static void ns_sweep_pairs(phl_ctx *c, hipStream_t s)
 {
     phl::DevFlow &f = c->f;
     const int nT = c->m.nTotal, nC = c->m.nCell;
-    hipMemsetAsync(f.dq, 0, sizeof(double) * phl::kRow * nT, s);
-    hipMemsetAsync(f.dflux, 0, sizeof(double) * phl::kRow * nC, s);
+    hipMemsetAsync(f.dflux, 0, sizeof(double) * 2 * phl::kPlanes * nC, s);
     hipMemsetAsync(f.dqPrev, 0, sizeof(double) * 5 * nC, s);
     double init = 0.0, eps = 1.1;
     c->nsLog.done = 0;
     for (int it = 0; it < c->k.nSweeps; ++it) {
         phl::launch_sweep(c->m, c->k, f, c->fwd, true, it == 0, s);
-        phl::launch_sweep_change(f.dq, phl::kRow, 1, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm, s);
+        phl::launch_sweep_change(f.dq, nT, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm, s);
         phl::launch_ghost_dq(c->m, c->k, f, s);
         phl::launch_sweep(c->m, c->k, f, c->bwd, false, false, s);
-        phl::launch_sweep_change(f.dq, phl::kRow, 1, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm + 1, s);
+        phl::launch_sweep_change(f.dq, nT, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm + 1, s);
         hipMemcpyAsync(c->nsLog.host, f.sweepNorm, 2 * sizeof(double), hipMemcpyDeviceToHost, s);
         if (hipStreamSynchronize(s) != hipSuccess) return;  // reported by the caller's launch check
         const double sn = c->nsLog.host[0] + c->nsLog.host[1];

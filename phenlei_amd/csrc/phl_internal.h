@@ -151,11 +151,11 @@ struct alignas(64) GatherRec {
 };
 static_assert(sizeof(GatherRec) == 192, "GatherRec is three 64-byte sectors");
 
-// The LU-SGS increments dq and off-diagonal sums are per-cell rows of kRow
-// doubles (one 64-byte line): a dataflow sweep reads a neighbour's five
-// increments with two 16-byte and one 8-byte device-scope load from one
-// line, and publishes its own with three such stores.
-constexpr int kRow = 8;
+// The LU-SGS increments dq and off-diagonal sums are rows of five values (a
+// sixth for the carried Spalart-Allmaras increment) in kPlanes planes of
+// 16-byte pairs, [kPlanes][rows][2]: a wavefront's access to a run of rows
+// is one contiguous 16-byte-per-lane access per plane.
+constexpr int kPlanes = 3;
 
 // Mutable flow state on the device.
 struct DevFlow {
@@ -168,11 +168,13 @@ struct DevFlow {
     float *gradTF;    // [3][nCell] mixed form
     double *lim;      // [nTotal]
     double *rtem;     // [nTotal] pressure factor (entropy fix 2, 6; null otherwise)
-    double *dq;       // [nTotal][kRow]: the five increments of a cell in one 64-byte line
-    double *dflux;    // [nCell][kRow]: the off-diagonal sums of the last sweep
+    double *dq;       // the increments of the last sweep: nTotal rows in pair planes (kPlanes)
+    double *dqAlt;    // dataflow sweeps: the buffer of the next sweep, every real row marked "not swept"
+                      // (a sweep swaps the two; null when neither direction has a dataflow order)
+    bool bwdFlow;     // the backward sweep is a dataflow sweep: ghost increments go to dqAlt
+    double *dflux;    // the off-diagonal sums of the last sweep: nCell rows in pair planes
     double *casePart; // batched contexts: [nCases][32][6] partial residual sums and dt minima
-    int *sweepFlag;   // [chunks] dataflow sweep: epoch of the sweep that last published the chunk's dq
-    int *sweepCtl;    // [4] dataflow sweep: ticket, epoch, waves that gave up waiting
+    int *sweepCtl;    // [4] dataflow sweep: ticket, unused, waves that gave up waiting, wait bound
     double *specInv, *specVis, *dtLoc, *dt, *diag;  // [nCell]
     double *normPart;   // [nBlocksFlux][5]
     double *normOut;    // [maxSteps][nCases][5], row = *stepCtr
@@ -224,12 +226,13 @@ struct SweepOrder {
 // depends only on chunks of earlier levels.
 struct FlowOrder {
     int nChunks;        // 0: not built
+    int W;              // slots per position: 3, 4 or 6
     const int *cells;   // [64*nChunks] storage index, -1 for padding
-    const int *row;     // [Wpad][64*nChunks] as SweepOrder::row
-    const int *nb;      // [Wpad][64*nChunks] as SweepOrder::nb
-    const int *depPtr;  // [nChunks+1]
-    const int *dep;     // the distinct earlier chunks holding a chunk's real neighbours
+    const int *row;     // [W][64*nChunks] as SweepOrder::row, real neighbours only
+    const int *nb;      // [W][64*nChunks] as SweepOrder::nb
     const int *width;   // [nChunks] most active slots of any cell of the chunk (slots are packed first)
+    const int *rowG;    // [most][64*nChunks] rows of the boundary faces (backward sweep; -1 pad), or null
+    const int *widthG;  // [nChunks] most boundary faces of any cell of the chunk
     // sweep_form 3: block i sweeps chunk blockChunk[i] (-1: nothing).  Each
     // level's chunks are split into 8 contiguous groups, group x going to the
     // blocks i = x (mod 8) of the level's block range, so that the k-th XCD
@@ -298,6 +301,7 @@ void launch_dt_diag(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s
 // before the forward one, launch_sa_ghost_dq between, launch_sa_update after).
 void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool forward,
                   bool firstSweep, hipStream_t s, bool withSA = false);
+void launch_mark_dq(const DevMesh &m, double *dq, hipStream_t s);
 void launch_ghost_dq(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s);
 void launch_update(const DevMesh &m, const Consts &k, DevFlow &f, bool advance, hipStream_t s);
 void launch_copy(const double *src, double *dst, size_t n, hipStream_t s);
@@ -305,8 +309,9 @@ void launch_forces(const DevMesh &m, const Consts &k, DevFlow &f, const double *
 
 // Spalart-Allmaras (phl_sa.hip).  tri: [nTri][9] wall triangles (face centre
 // and two consecutive face nodes).
-void launch_sweep_change(const double *dq, size_t cs, size_t ms, int nv, int nC, double *prev, double *parts,
-                         double *out, hipStream_t s);
+// nv 5: dq in pair planes of n rows; nv 1: a plain array.
+void launch_sweep_change(const double *dq, int n, int nv, int nC, double *prev, double *parts, double *out,
+                         hipStream_t s);
 void launch_wall_distance(const double *xcc, const double *ycc, const double *zcc, int nCell, const double *tri,
                           int nTri, bool edges, double *wd, hipStream_t s);
 void launch_sa_boundary(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s);

@@ -245,21 +245,37 @@ __device__ __forceinline__ void load5(const double *__restrict__ a, int n, int i
     for (int m = 0; m < 5; ++m) v[m] = a[(size_t)m * n + i];
 }
 
-// The first five values of row i of a [n][kRow] array (one 64-byte line).
-__device__ __forceinline__ void load_row5(const double *a, int i, double *v)
+// The five values of row i of an n-row array in pair planes (kPlanes).
+__device__ __forceinline__ double2 *pair_at(double *a, int n, int i, int plane)
 {
-    const double *r = a + (size_t)i * kRow;
-    const double2 x = *reinterpret_cast<const double2 *>(r);
-    const double2 y = *reinterpret_cast<const double2 *>(r + 2);
-    v[0] = x.x; v[1] = x.y; v[2] = y.x; v[3] = y.y; v[4] = r[4];
+    return reinterpret_cast<double2 *>(a) + (size_t)plane * n + i;
+}
+__device__ __forceinline__ const double2 *pair_at(const double *a, int n, int i, int plane)
+{
+    return reinterpret_cast<const double2 *>(a) + (size_t)plane * n + i;
 }
 
-__device__ __forceinline__ void store_row5(double *a, int i, const double *v)
+__device__ __forceinline__ void load_row5(const double *a, int n, int i, double *v)
 {
-    double *r = a + (size_t)i * kRow;
-    *reinterpret_cast<double2 *>(r) = make_double2(v[0], v[1]);
-    *reinterpret_cast<double2 *>(r + 2) = make_double2(v[2], v[3]);
-    r[4] = v[4];
+    const double2 x = *pair_at(a, n, i, 0), y = *pair_at(a, n, i, 1);
+    v[0] = x.x; v[1] = x.y; v[2] = y.x; v[3] = y.y; v[4] = pair_at(a, n, i, 2)->x;
+}
+
+__device__ __forceinline__ void store_row5(double *a, int n, int i, const double *v)
+{
+    *pair_at(a, n, i, 0) = make_double2(v[0], v[1]);
+    *pair_at(a, n, i, 1) = make_double2(v[2], v[3]);
+    pair_at(a, n, i, 2)->x = v[4];
+}
+
+// The "not swept yet" mark of an increment (all bits set, a NaN that no
+// arithmetic of the hardware produces), and a value made distinct from it (a
+// NaN payload carried in from the caller's state).
+constexpr unsigned long long kMark = ~0ull;
+__device__ __forceinline__ bool is_mark(double v) { return (unsigned long long)__double_as_longlong(v) == kMark; }
+__device__ __forceinline__ double not_mark(double v)
+{
+    return is_mark(v) ? __longlong_as_double(0x7ff8000000000000ll) : v;
 }
 
 // ------------------------------------------------------------------ BCs
@@ -1671,23 +1687,25 @@ __global__ void __launch_bounds__(kBlock) k_norm_sum5(const double *__restrict__
 // The squared change of dq since the last call (the sweepNormal of
 // Controller::LUSGS for nLUSGSSweeps > 1, Controller.cpp:1920-1950; the
 // reference adds SQR(dq - dqOld) cell by cell in its sweeps): per block of
-// kBlock real cells, over nv components (component m of cell c at
-// dq[c * cs + m * ms]), and prev [nv][nC] takes the new dq.  k_sum_into then
-// adds the block partials in a fixed order.
-__global__ void __launch_bounds__(kBlock) k_sweep_change(const double *__restrict__ dq, size_t cs, size_t ms, int nv,
-                                                         int nC, double *__restrict__ prev,
-                                                         double *__restrict__ parts)
+// kBlock real cells, over nv components (5: pair planes of n rows; 1: a plain
+// array), and prev [nv][nC] takes the new dq.  k_sum_into then adds the block
+// partials in a fixed order.
+__global__ void __launch_bounds__(kBlock) k_sweep_change(const double *__restrict__ dq, int n, int nv, int nC,
+                                                         double *__restrict__ prev, double *__restrict__ parts)
 {
     __shared__ double red[kBlock];
     const int c = blockIdx.x * kBlock + (int)threadIdx.x;
     double acc = 0.0;
-    if (c < nC)
+    if (c < nC) {
+        double v[5];
+        if (nv == 5) load_row5(dq, n, c, v);
+        else v[0] = dq[c];
         for (int m = 0; m < nv; ++m) {
-            const double v = dq[(size_t)c * cs + (size_t)m * ms];
-            const double d = v - prev[(size_t)m * nC + c];
+            const double d = v[m] - prev[(size_t)m * nC + c];
             acc += d * d;
-            prev[(size_t)m * nC + c] = v;
+            prev[(size_t)m * nC + c] = v[m];
         }
+    }
     red[threadIdx.x] = acc;
     __syncthreads();
     for (int w = kBlock / 2; w > 0; w >>= 1) {
@@ -1839,15 +1857,15 @@ __device__ __forceinline__ void sweep_finish(const DevMesh &M, int c, bool useU,
     double r[5], U[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     load5(res, nC, c, r);
     const double D = diag[c];
-    if (useU) load_row5(dflux, c, U);
+    if (useU) load_row5(dflux, M.nCell, c, U);
     double v[5], w[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         v[m] = (r[m] - U[m] - rhs0[m]) / D;
         w[m] = 0.0 + rhs0[m];
     }
-    store_row5(dq, c, v);
-    store_row5(dflux, c, w);
+    store_row5(dq, M.nTotal, c, v);
+    store_row5(dflux, M.nCell, c, w);
 }
 
 __device__ __forceinline__ void load_coef(const double *__restrict__ coef, int f, bool isL, double *co)
@@ -1891,7 +1909,7 @@ __device__ __forceinline__ void sweep_cell_batched(const DevMesh &M, const Const
         const bool isL = enc[s] > 0;
         const int f = act[s] ? (isL ? enc[s] : -enc[s]) - 1 : 0;
         load_coef(coef, f, isL, co[s]);
-        load_row5(dq, act[s] ? nb[s] : 0, dqn[s]);
+        load_row5(dq, M.nTotal, act[s] ? nb[s] : 0, dqn[s]);
     }
     double rhs0[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -1922,7 +1940,7 @@ __device__ __forceinline__ void sweep_cell_generic(const DevMesh &M, const Const
         const int f = (isL ? enc : -enc) - 1;
         double co[15], dqn[5], df[5];
         load_coef(coef, f, isL, co);
-        load_row5(dq, nb, dqn);
+        load_row5(dq, M.nTotal, nb, dqn);
         sweep_apply(K, co, dqn, df);
 #pragma unroll
         for (int m = 0; m < 5; ++m) rhs0[m] += df[m];
@@ -2011,13 +2029,13 @@ __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K
     double r[5], U[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     load5(res, P, c, r);
     const double D = diag[c];
-    if (useU) load_row5(dflux, c, U);
+    if (useU) load_row5(dflux, M.nCell, c, U);
     double co[NW][16], dqn[NW][5];
 #pragma unroll
     for (int s = 0; s < NW; ++s) {
         const bool act = row[s] >= 0;
         load_coef_row<CT>(coef, act ? row[s] : 0, co[s]);
-        load_row5(dq, act ? nb[s] : 0, dqn[s]);
+        load_row5(dq, M.nTotal, act ? nb[s] : 0, dqn[s]);
     }
     // Unused slots add +0.0, which leaves the sum unchanged (it starts at
     // +0.0, so it is never -0.0); no branch lets the loads of a slot sink.
@@ -2036,8 +2054,8 @@ __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K
         v[m] = (r[m] - U[m] - rhs0[m]) / D;
         w[m] = 0.0 + rhs0[m];
     }
-    store_row5(dq, c, v);
-    store_row5(dflux, c, w);
+    store_row5(dq, M.nTotal, c, v);
+    store_row5(dflux, M.nCell, c, w);
 }
 
 template <int NW, int VIS, typename CT>
@@ -2066,19 +2084,33 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_block_so(DevMesh M, Const
 }
 
 // ------------------------------------------------- dataflow sweep
-// One launch per direction instead of one per level (sweep_form 0 and 2).  Each
-// 64-thread block (one wavefront) takes the next chunk of 64 positions of
-// the padded level order from a ticket counter.  A chunk depends only on
-// chunks of earlier levels, which were taken earlier by blocks that are
-// running or done, so every wait ends.  The wave polls the flags of the
-// chunks it depends on (one per lane), then sweeps its 64 cells exactly as
-// sweep_position does and publishes its chunk.  dq and the flags are stored
-// and loaded with device-scope (sc1) accesses, which are coherent across the
-// XCDs' L2 caches, and the wave's dq stores complete (vmcnt 0) before its
-// flag store is issued.
-// ctl: [0] ticket, [1] epoch of the current sweep, [2] waves that gave up,
-// [3] the wait bound in ticks of the 100 MHz wall clock (set by the host;
-// 20,000,000 = 0.2 s by default).
+// One launch per direction instead of one per level (sweep_form 0, 2 and 3).
+// A wavefront sweeps one chunk of 64 positions of the padded level order; a
+// chunk depends only on chunks of earlier levels, which earlier blocks hold.
+//
+// The increments themselves say when they are there.  Every sweep writes the
+// one of two dq buffers that holds kMark in every real row, and marks the
+// rows of the other (whose last reader has run) for the next sweep; a wave
+// loads its neighbours' rows and loads those again that still hold a mark.
+// Each 8-byte value carries its own mark, so no order between the stores of a
+// row is assumed.  dq is stored and loaded with device-scope (sc1) accesses,
+// which are coherent across the XCDs' L2 caches.
+//
+// Bound: the chain of levels.  A level costs one store-to-load propagation
+// (0.85 us between two idle waves; 1.66 us with an acknowledged store, a flag
+// and the dq loads after it) plus the arithmetic of one wavefront.  Per step,
+// forward + backward, per-chunk flags published after the acknowledgement
+// took 1.53 + 1.56 ms on the 2.24M-cell wing, 0.99 + 0.99 on the 1.01M-cell
+// hybrid channel, 0.60 + 0.63 on the 254k-cell and 0.23 + 0.27 on the 16k-cell
+// hex channel; marks take 0.90 + 1.04, 0.55 + 0.57, 0.50 + 0.50 and 0.20 +
+// 0.20.  A flag published early as a hint, before polling the rows, was slower
+// than polling at once (wing 1.10 + 1.22).
+// Polling the rows pays only because they are few lines: storage follows the
+// level order (sweep_order), so the 64 neighbours of a slot lie in short runs
+// of rows, and the pair planes (kPlanes) keep a run contiguous.
+// ctl: [0] ticket (sweep_form 2), [2] waves that gave up, [3] the wait bound
+// in ticks of the 100 MHz wall clock (set by the host; 20,000,000 = 0.2 s by
+// default).
 
 // 128- and 64-bit payloads of the raw buffer loads and stores, and word 3
 // of their buffer descriptor (untyped 32-bit data, as raw buffer accesses
@@ -2087,34 +2119,54 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 constexpr int kRawBufferWord3 = 0x00020000;
 constexpr int kDeviceScope = 16;
-__global__ void k_sweep_flow_prep(int *ctl)
-{
-    ctl[0] = 0;
-    ctl[1] += 1;
-}
+__global__ void k_sweep_ticket(int *ctl) { ctl[0] = 0; }
 
-__device__ __forceinline__ int flag_load(const int *p)
+__device__ __forceinline__ int ctl_load(const int *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ double dq_load(const double *p)
+// Both dq buffers' marks: all n values of an array.
+__global__ void __launch_bounds__(kBlock) k_mark(unsigned long long *__restrict__ a, size_t n)
 {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = kMark;
+}
+
+// The coefficients of face side `rw` of cell cc (state qc, centroid xc, eddy
+// viscosity vc) towards neighbour n, as k_grad_lim evaluates them for the
+// level form: sweep_coef on the same operands, rounded to CT as a stored row
+// is.  The neighbour's state and centroid come from its gather record (the
+// first 64 bytes: one line instead of eight).
+template <typename CT>
+__device__ __forceinline__ void side_coef(const DevMesh &M, const Consts &Kc, const GatherRec *__restrict__ rec,
+                                          const double *__restrict__ vist, const double *qc, const double *xc,
+                                          double vc, int rw, int n, double *co)
+{
+    const FaceRec fr = M.face[rw >> 1];
+    double qn[5], xn[3];
+    load_rec_state(rec, n, qn, xn);
+    const double dist = Kc.viscous ? dABS(fr.nx * (xn[0] - xc[0]) + fr.ny * (xn[1] - xc[1]) + fr.nz * (xn[2] - xc[2]))
+                                   : 0.0;
+    sweep_coef(Kc, qc, qn, fr, (rw & 1) == 0, dist, vc, vist[n], co);
+    if constexpr (sizeof(CT) == 4) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) co[j] = double(float(co[j]));
+    }
 }
 
 // One chunk of the dataflow sweep, swept by one wavefront: false if the wait
 // bound was exceeded (the chunk is then neither swept nor published).
 // sa.on: the chunk's cells also take the same-direction step of the scalar
-// Spalart-Allmaras sweep (the same lists and order as sa_sweep_position; its
-// dq is published under the same flag).
+// Spalart-Allmaras sweep (the same lists and order as sa_sweep_position);
+// its increment is the sixth value of a dq row.
 template <int NW, int VIS, typename CT>
-__device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, const FlowOrder &fo, int *ctl,
-                                           int *chunkFlag, bool useU, const double *__restrict__ coef,
+__device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, const FlowOrder &fo, const int *ctl,
+                                           bool useU, const double *__restrict__ coef,
                                            const double *__restrict__ res, const double *__restrict__ diag,
-                                           double *dq, double *dflux, const SaSweep &sa,
+                                           double *dq, double *dqOld, double *dflux, const SaSweep &sa,
                                            const GatherRec *__restrict__ rec, const double *__restrict__ vist, int tk,
-                                           int lane, int epoch, long long t0, long long waitTicks)
+                                           int lane, long long t0, long long waitTicks)
 {
     const int nT = M.nTotal, nC = M.nCell, P = 64 * fo.nChunks;
     const int p = tk * 64 + lane;
@@ -2140,33 +2192,19 @@ __device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, co
     load5(res, nC, cc, r);
     const double D = diag[cc];
     double U[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (useU) load_row5(dflux, cc, U);
+    if (useU) load_row5(dflux, nC, cc, U);
     double co[NW][16];
+    Consts Kc = K;
+    double qc[5], xc[3], vc = 0.0;
     if (K.coefInSweep) {
-        // the face terms of k_grad_lim, evaluated here while the chunk waits:
-        // sweep_coef on the same operands, rounded to CT as a stored row is.
-        // States and centroids come from the gather records (the first 64
-        // bytes of a record: one line per neighbour instead of eight).
-        const Consts Kc = case_k(K, M, cc);
-        double qc[5], xc[3];
+        Kc = case_k(K, M, cc);
         load_rec_state(rec, cc, qc, xc);
-        const double vc = vist[cc];
+        vc = vist[cc];
 #pragma unroll
         for (int s = 0; s < NW; ++s) {
             if (s >= width) break;
             const int rw = row[s] >= 0 ? row[s] : 0, n = row[s] >= 0 ? nb[s] : cc;
-            const FaceRec fr = M.face[rw >> 1];
-            const bool isL = (rw & 1) == 0;
-            double qn[5], xn[3];
-            load_rec_state(rec, n, qn, xn);
-            const double dist = Kc.viscous ? dABS(fr.nx * (xn[0] - xc[0]) + fr.ny * (xn[1] - xc[1]) +
-                                                  fr.nz * (xn[2] - xc[2]))
-                                           : 0.0;
-            sweep_coef(Kc, qc, qn, fr, isL, dist, vc, vist[n], co[s]);
-            if constexpr (sizeof(CT) == 4) {
-#pragma unroll
-                for (int j = 0; j < 16; ++j) co[s][j] = double(float(co[s][j]));
-            }
+            side_coef<CT>(M, Kc, rec, vist, qc, xc, vc, rw, n, co[s]);
         }
     } else {
 #pragma unroll
@@ -2181,99 +2219,108 @@ __device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, co
         DT = sa.spec[cc];
         UT = sa.dflux[cc];
     }
-
-    // wait for the chunks this one depends on, one flag per lane
-    const int d0 = fo.depPtr[tk], d1 = fo.depPtr[tk + 1];
-    for (int i0 = d0; i0 < d1; i0 += 64) {
-        const int i = i0 + lane;
-        bool ok = i >= d1;
-        const int dc = ok ? 0 : fo.dep[i];
-        for (int it = 1;; ++it) {
-            if (!ok) ok = flag_load(&chunkFlag[dc]) == epoch;
-            if (__all(ok)) break;
-            // bounded wait: never reached by a correct schedule; a wave that
-            // gives up makes every later waiter give up too
-            if (wall_clock64() - t0 > waitTicks || ((it & 63) == 0 && flag_load(&ctl[2]) != 0)) return false;
-            __builtin_amdgcn_s_sleep(1);
-        }
+    const __amdgpu_buffer_rsrc_t dqr = __builtin_amdgcn_make_buffer_rsrc(
+        dq, 0, (int)((size_t)nT * kPlanes * sizeof(double2)), kRawBufferWord3);
+    const int plane = nT * (int)sizeof(double2);
+    // Terms of ghost neighbours (backward sweep): boundary faces precede
+    // every interior face, so they come first in a cell's sum, and the ghost
+    // kernel has written their dq before this launch.  Few chunks have any;
+    // kept out of the polled slots they leave a hex backward sweep three
+    // slots instead of six (16k cells: 0.30 -> 0.20 ms).
+    double rhs0[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, rhsT = 0.0;
+    const int widthG = fo.rowG ? __builtin_amdgcn_readfirstlane(fo.widthG[tk]) : 0;
+    for (int s = 0; s < widthG; ++s) {
+        const int rw = fo.rowG[(size_t)s * P + p];
+        if (rw < 0) continue;
+        const int g = nC + (rw >> 1);
+        double cg[16], dg[5], df[5];
+        if (K.coefInSweep) side_coef<CT>(M, Kc, rec, vist, qc, xc, vc, rw, g, cg);
+        else load_coef_row<CT>(coef, rw, cg);
+        load_row5(dq, nT, g, dg);
+        sweep_apply<VIS>(K, cg, dg, df);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) rhs0[m] += df[m];
+        if (sa.on) rhsT += sa.mat[rw] * pair_at(dq, nT, g, 2)->y;
     }
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);  // the dq loads stay after the flag loads
-    double dqn[NW][5], dT[NW];
+
+    // the neighbours' increments, loaded until none is marked (the lanes and
+    // slots that have theirs keep them in place)
+    v4i x[NW], y[NW], z[NW];
+    bool wait[NW];
 #pragma unroll
     for (int s = 0; s < NW; ++s) {
-        dT[s] = 0.0;
-        if (s >= width) break;
-        const int i = row[s] >= 0 ? nb[s] : 0;
-        // the neighbour's row with device-scope (sc1) vector loads: three
-        // requests to one line instead of five 8-byte loads; with the SA
-        // sweep carried, the row's slot 5 holds the neighbour's nu~ increment
-        {
-            const __amdgpu_buffer_rsrc_t dqr =
-                __builtin_amdgcn_make_buffer_rsrc(dq, 0, (int)((size_t)nT * kRow * sizeof(double)), kRawBufferWord3);
-            const v4i a = __builtin_amdgcn_raw_buffer_load_b128(dqr, i * kRow * 8, 0, kDeviceScope);
-            const v4i b = __builtin_amdgcn_raw_buffer_load_b128(dqr, i * kRow * 8 + 16, 0, kDeviceScope);
-            const double2 da = __builtin_bit_cast(double2, a), db = __builtin_bit_cast(double2, b);
-            dqn[s][0] = da.x; dqn[s][1] = da.y; dqn[s][2] = db.x; dqn[s][3] = db.y;
-            if (sa.on) {
-                const double2 dc = __builtin_bit_cast(
-                    double2, __builtin_amdgcn_raw_buffer_load_b128(dqr, i * kRow * 8 + 32, 0, kDeviceScope));
-                dqn[s][4] = dc.x;
-                dT[s] = dc.y;
-            } else {
-                dqn[s][4] = __builtin_bit_cast(
-                    double, __builtin_amdgcn_raw_buffer_load_b64(dqr, i * kRow * 8 + 32, 0, kDeviceScope));
+        wait[s] = row[s] >= 0;
+        x[s] = y[s] = z[s] = v4i{0, 0, 0, 0};
+    }
+    for (int it = 1;; ++it) {
+#pragma unroll
+        for (int s = 0; s < NW; ++s) {
+            if (s >= width) break;
+            if (wait[s]) {
+                const int o = nb[s] * (int)sizeof(double2);
+                x[s] = __builtin_amdgcn_raw_buffer_load_b128(dqr, o, 0, kDeviceScope);
+                y[s] = __builtin_amdgcn_raw_buffer_load_b128(dqr, o + plane, 0, kDeviceScope);
+                z[s] = __builtin_amdgcn_raw_buffer_load_b128(dqr, o + 2 * plane, 0, kDeviceScope);
             }
         }
+        bool again = false;
+#pragma unroll
+        for (int s = 0; s < NW; ++s) {
+            if (s >= width) break;
+            // bitwise and: one test of a pair of words per value
+            wait[s] = wait[s] && (((x[s][0] & x[s][1]) == -1) | ((x[s][2] & x[s][3]) == -1) |
+                                  ((y[s][0] & y[s][1]) == -1) | ((y[s][2] & y[s][3]) == -1) |
+                                  ((z[s][0] & z[s][1]) == -1) | (sa.on & ((z[s][2] & z[s][3]) == -1)));
+            again = again || wait[s];
+        }
+        if (!__any(again)) break;
+        // bounded wait: never reached by a correct schedule; a wave that
+        // gives up makes every later waiter give up too
+        if (wall_clock64() - t0 > waitTicks || ((it & 63) == 0 && ctl_load(&ctl[2]) != 0)) return false;
+        __builtin_amdgcn_s_sleep(1);
     }
-    double rhs0[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int s = 0; s < NW; ++s) {
         if (s >= width) break;
+        const double2 a = __builtin_bit_cast(double2, x[s]), b = __builtin_bit_cast(double2, y[s]),
+                      d = __builtin_bit_cast(double2, z[s]);
+        const double dqn[5] = {a.x, a.y, b.x, b.y, d.x};
         double df[5];
-        sweep_apply<VIS>(K, co[s], dqn[s], df);
+        sweep_apply<VIS>(K, co[s], dqn, df);
         const bool act = row[s] >= 0;
 #pragma unroll
         for (int m = 0; m < 5; ++m) rhs0[m] += act ? df[m] : 0.0;
-    }
-    double rhsT = 0.0;
-    if (sa.on) {
-#pragma unroll
-        for (int s = 0; s < NW; ++s)
-            if (s < width) rhsT += (row[s] >= 0) ? aT[s] * dT[s] : 0.0;
+        if (sa.on) rhsT += act ? aT[s] * d.y : 0.0;
     }
     if (live) {
-        // the cell's row with device-scope (sc1) vector stores
         double v[5];
 #pragma unroll
-        for (int m = 0; m < 5; ++m) v[m] = (r[m] - U[m] - rhs0[m]) / D;
-        const __amdgpu_buffer_rsrc_t dqw =
-            __builtin_amdgcn_make_buffer_rsrc(dq, 0, (int)((size_t)nT * kRow * sizeof(double)), kRawBufferWord3);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_double2(v[0], v[1])), dqw, c * kRow * 8, 0,
+        for (int m = 0; m < 5; ++m) v[m] = not_mark((r[m] - U[m] - rhs0[m]) / D);
+        const double vT = sa.on ? not_mark((rT - UT - rhsT) / DT) : 0.0;
+        const int o = c * (int)sizeof(double2);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_double2(v[0], v[1])), dqr, o, 0,
                                                kDeviceScope);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_double2(v[2], v[3])), dqw,
-                                               c * kRow * 8 + 16, 0, kDeviceScope);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_double2(v[2], v[3])), dqr, o + plane, 0,
+                                               kDeviceScope);
         if (sa.on)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_double2(v[4], (rT - UT - rhsT) / DT)),
-                                                   dqw, c * kRow * 8 + 32, 0, kDeviceScope);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_double2(v[4], vT)), dqr,
+                                                   o + 2 * plane, 0, kDeviceScope);
         else
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, v[4]), dqw, c * kRow * 8 + 32, 0,
-                                                  kDeviceScope);
-    }
-    // the wave's dq stores are complete before the flag that publishes them
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    if (lane == 0) __hip_atomic_store(&chunkFlag[tk], epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the off-diagonal sums are read only by the next sweep (another launch)
-    if (live) {
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, v[4]), dqr, o + 2 * plane, 0, kDeviceScope);
+        // the rest is read only by later launches: the off-diagonal sums, the
+        // SA increment's plain array (ghost, update and field kernels), and
+        // the marks of the other buffer for the next sweep
         double w[5];
 #pragma unroll
         for (int m = 0; m < 5; ++m) w[m] = 0.0 + rhs0[m];
-        store_row5(dflux, c, w);
+        store_row5(dflux, nC, c, w);
         if (sa.on) {
             sa.dflux[c] = 0.0 + rhsT;
-            sa.dq[c] = (rT - UT - rhsT) / DT;  // for the ghost, update and field kernels
+            sa.dq[c] = vT;
         }
+        const double mark = __longlong_as_double((long long)kMark);
+#pragma unroll
+        for (int m = 0; m < kPlanes; ++m) *pair_at(dqOld, nT, c, m) = make_double2(mark, mark);
     }
     return true;
 }
@@ -2290,10 +2337,9 @@ __device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, co
 // is one device-scope atomic per block, which serialises large launches).
 template <int NW, int VIS, typename CT, bool TICKET>
 __global__ void __launch_bounds__(TICKET ? 256 : 64) k_sweep_flow(DevMesh M, Consts K, FlowOrder fo, int *ctl,
-                                                                  int *chunkFlag, bool useU,
-                                                                  const double *__restrict__ coef,
+                                                                  bool useU, const double *__restrict__ coef,
                                                                   const double *__restrict__ res, const double *__restrict__ diag, double *dq,
-                                                                  double *dflux, SaSweep sa,
+                                                                  double *dqOld, double *dflux, SaSweep sa,
                                                                   const GatherRec *__restrict__ rec,
                                                                   const double *__restrict__ vist)
 {
@@ -2311,13 +2357,15 @@ __global__ void __launch_bounds__(TICKET ? 256 : 64) k_sweep_flow(DevMesh M, Con
     } else {
         tk = blockIdx.x;
     }
-    if (!flow_chunk<NW, VIS, CT>(M, K, fo, ctl, chunkFlag, useU, coef, res, diag, dq, dflux, sa, rec, vist, tk, lane,
-                                 ctl[1], wall_clock64(), (long long)ctl[3]))
+    if (!flow_chunk<NW, VIS, CT>(M, K, fo, ctl, useU, coef, res, diag, dq, dqOld, dflux, sa, rec, vist, tk, lane,
+                                 wall_clock64(), (long long)ctl[3]))
         if (lane == 0) atomicAdd(&ctl[2], 1);
 }
 
+// Ghost dq from the forward sweep's dq, into the buffer the backward sweep
+// will use (`out`; the same one in the level form).
 __global__ void __launch_bounds__(kBlock) k_ghost_dq(DevMesh M, Consts K, const double *__restrict__ q,
-                                                     double *__restrict__ dq)
+                                                     const double *dq, double *out)
 {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= M.nBFace) return;
@@ -2325,7 +2373,7 @@ __global__ void __launch_bounds__(kBlock) k_ghost_dq(DevMesh M, Consts K, const 
     const int le = M.fle[f], re = M.nCell + f;
     const int bc = M.bcType[f];
     double dl[5], dr[5];
-    load_row5(dq, le, dl);
+    load_row5(dq, nT, le, dl);
     if (bc == kBC_SYMM || (bc == kBC_WALL && !K.viscous)) {
         double prim[5], Q[5];
         load5(q, nT, le, prim);
@@ -2364,7 +2412,9 @@ __global__ void __launch_bounds__(kBlock) k_ghost_dq(DevMesh M, Consts K, const 
 #pragma unroll
         for (int m = 0; m < 5; ++m) dr[m] = 0.0;
     }
-    store_row5(dq, re, dr);
+#pragma unroll
+    for (int m = 0; m < 5; ++m) dr[m] = not_mark(dr[m]);
+    store_row5(out, nT, re, dr);
 }
 
 // ------------------------------------------------------------- update
@@ -2389,7 +2439,7 @@ __global__ void __launch_bounds__(kBlock) k_update(DevMesh M, Consts K0, const d
         Q[0] = prim[0]; Q[1] = prim[0] * prim[1]; Q[2] = prim[0] * prim[2]; Q[3] = prim[0] * prim[3];
         Q[4] = prim[0] * em;
         double d5[5];
-        load_row5(dq, i, d5);
+        load_row5(dq, nT, i, d5);
 #pragma unroll
         for (int m = 0; m < 5; ++m) Q[m] += d5[m];
         if (Q[0] <= 0.0) {
@@ -2857,25 +2907,49 @@ void launch_dt_diag(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s
 // (barriers are cheap); larger levels are spread over the GPU.
 static const int kSmallLevel = kSweepBlock;
 
+// Marks every row of a dq buffer (the next dataflow sweep's).
+void launch_mark_dq(const DevMesh &m, double *dq, hipStream_t s)
+{
+    const size_t n = (size_t)2 * kPlanes * m.nTotal;
+    hipLaunchKernelGGL(k_mark, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
+                       reinterpret_cast<unsigned long long *>(dq), n);
+}
+
+template <int NW, int VIS, typename CT>
+static void launch_sweep_flow(const DevMesh &m, const Consts &k, DevFlow &f, const FlowOrder &fo, bool useU,
+                              bool withSA, hipStream_t s)
+{
+    SaSweep sa{};
+    if (withSA) sa = SaSweep{true, f.saMat, f.resT, f.specT, f.dqT, f.dfluxT};
+    std::swap(f.dq, f.dqAlt);  // the marked buffer becomes the current one
+    if (k.sweepForm == 2) {
+        hipLaunchKernelGGL(k_sweep_ticket, dim3(1), dim3(1), 0, s, f.sweepCtl);
+        hipLaunchKernelGGL((k_sweep_flow<NW, VIS, CT, true>), dim3(nblk(fo.nChunks, 4)), dim3(256), 0, s, m, k, fo,
+                           f.sweepCtl, useU, f.coef, f.res, f.diag, f.dq, f.dqAlt, f.dflux, sa, f.rec, f.vist);
+    } else {
+        hipLaunchKernelGGL((k_sweep_flow<NW, VIS, CT, false>), dim3(k.sweepForm == 3 ? fo.nBlocks : fo.nChunks),
+                           dim3(64), 0, s, m, k, fo, f.sweepCtl, useU, f.coef, f.res, f.diag, f.dq, f.dqAlt, f.dflux,
+                           sa, f.rec, f.vist);
+    }
+}
+
+template <int NW>
+static void launch_sweep_flow_w(const DevMesh &m, const Consts &k, DevFlow &f, const FlowOrder &fo, bool useU,
+                                bool withSA, hipStream_t s)
+{
+    if (k.coefF32) {  // only set when both directions have at most 6 slots
+        if (k.viscous) launch_sweep_flow<NW, 1, float>(m, k, f, fo, useU, withSA, s);
+        else launch_sweep_flow<NW, 0, float>(m, k, f, fo, useU, withSA, s);
+    } else {
+        if (k.viscous) launch_sweep_flow<NW, 1, double>(m, k, f, fo, useU, withSA, s);
+        else launch_sweep_flow<NW, 0, double>(m, k, f, fo, useU, withSA, s);
+    }
+}
+
 template <int NW, int VIS, typename CT>
 static void launch_sweep_so(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool useU,
-                            bool withSA, hipStream_t s)
+                            hipStream_t s)
 {
-    if (lv.flow.nChunks > 0) {  // built unless sweep_form is 1
-        SaSweep sa{};
-        if (withSA) sa = SaSweep{true, f.saMat, f.resT, f.specT, f.dqT, f.dfluxT};
-        hipLaunchKernelGGL(k_sweep_flow_prep, dim3(1), dim3(1), 0, s, f.sweepCtl);
-        if (k.sweepForm == 2)
-            hipLaunchKernelGGL((k_sweep_flow<NW, VIS, CT, true>), dim3(nblk(lv.flow.nChunks, 4)), dim3(256), 0, s, m,
-                               k, lv.flow, f.sweepCtl, f.sweepFlag, useU, f.coef, f.res, f.diag, f.dq, f.dflux, sa,
-                               f.rec, f.vist);
-        else
-            hipLaunchKernelGGL((k_sweep_flow<NW, VIS, CT, false>),
-                               dim3(k.sweepForm == 3 ? lv.flow.nBlocks : lv.flow.nChunks), dim3(64), 0, s, m, k,
-                               lv.flow, f.sweepCtl, f.sweepFlag, useU, f.coef, f.res, f.diag, f.dq, f.dflux, sa,
-                               f.rec, f.vist);
-        return;
-    }
     int L = 0;
     while (L < lv.nLevels) {
         const int sz = lv.hptr[L + 1] - lv.hptr[L];
@@ -2898,14 +2972,19 @@ void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &l
 {
     const bool useU = !(forward && firstSweep);
     const bool v = k.viscous != 0;
-    if (k.coefF32) {  // only set when both directions have at most 6 slots
-        if (lv.so.Wpad == 3) return v ? launch_sweep_so<3, 1, float>(m, k, f, lv, useU, withSA, s) : launch_sweep_so<3, 0, float>(m, k, f, lv, useU, withSA, s);
-        if (lv.so.Wpad == 4) return v ? launch_sweep_so<4, 1, float>(m, k, f, lv, useU, withSA, s) : launch_sweep_so<4, 0, float>(m, k, f, lv, useU, withSA, s);
-        return v ? launch_sweep_so<6, 1, float>(m, k, f, lv, useU, withSA, s) : launch_sweep_so<6, 0, float>(m, k, f, lv, useU, withSA, s);
+    if (lv.flow.nChunks > 0) {  // built unless sweep_form is 1
+        if (lv.flow.W == 3) return launch_sweep_flow_w<3>(m, k, f, lv.flow, useU, withSA, s);
+        if (lv.flow.W == 4) return launch_sweep_flow_w<4>(m, k, f, lv.flow, useU, withSA, s);
+        return launch_sweep_flow_w<6>(m, k, f, lv.flow, useU, withSA, s);
     }
-    if (lv.so.Wpad == 3) return v ? launch_sweep_so<3, 1, double>(m, k, f, lv, useU, withSA, s) : launch_sweep_so<3, 0, double>(m, k, f, lv, useU, withSA, s);
-    if (lv.so.Wpad == 4) return v ? launch_sweep_so<4, 1, double>(m, k, f, lv, useU, withSA, s) : launch_sweep_so<4, 0, double>(m, k, f, lv, useU, withSA, s);
-    if (lv.so.Wpad == 6) return v ? launch_sweep_so<6, 1, double>(m, k, f, lv, useU, withSA, s) : launch_sweep_so<6, 0, double>(m, k, f, lv, useU, withSA, s);
+    if (k.coefF32) {
+        if (lv.so.Wpad == 3) return v ? launch_sweep_so<3, 1, float>(m, k, f, lv, useU, s) : launch_sweep_so<3, 0, float>(m, k, f, lv, useU, s);
+        if (lv.so.Wpad == 4) return v ? launch_sweep_so<4, 1, float>(m, k, f, lv, useU, s) : launch_sweep_so<4, 0, float>(m, k, f, lv, useU, s);
+        return v ? launch_sweep_so<6, 1, float>(m, k, f, lv, useU, s) : launch_sweep_so<6, 0, float>(m, k, f, lv, useU, s);
+    }
+    if (lv.so.Wpad == 3) return v ? launch_sweep_so<3, 1, double>(m, k, f, lv, useU, s) : launch_sweep_so<3, 0, double>(m, k, f, lv, useU, s);
+    if (lv.so.Wpad == 4) return v ? launch_sweep_so<4, 1, double>(m, k, f, lv, useU, s) : launch_sweep_so<4, 0, double>(m, k, f, lv, useU, s);
+    if (lv.so.Wpad == 6) return v ? launch_sweep_so<6, 1, double>(m, k, f, lv, useU, s) : launch_sweep_so<6, 0, double>(m, k, f, lv, useU, s);
     // wider polyhedra: face-by-face through the cell -> face lists
     int L = 0;
     while (L < lv.nLevels) {
@@ -2932,18 +3011,19 @@ void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &l
     }
 }
 
-void launch_sweep_change(const double *dq, size_t cs, size_t ms, int nv, int nC, double *prev, double *parts,
-                         double *out, hipStream_t s)
+void launch_sweep_change(const double *dq, int n, int nv, int nC, double *prev, double *parts, double *out,
+                         hipStream_t s)
 {
     const int nb = nblk(nC, kBlock);
-    hipLaunchKernelGGL(k_sweep_change, dim3(nb), dim3(kBlock), 0, s, dq, cs, ms, nv, nC, prev, parts);
+    hipLaunchKernelGGL(k_sweep_change, dim3(nb), dim3(kBlock), 0, s, dq, n, nv, nC, prev, parts);
     hipLaunchKernelGGL(k_sum_into, dim3(1), dim3(kBlock), 0, s, parts, nb, out);
 }
 
 void launch_ghost_dq(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s)
 {
     if (m.nBFace == 0) return;
-    hipLaunchKernelGGL(k_ghost_dq, dim3(nblk(m.nBFace, kBlock)), dim3(kBlock), 0, s, m, k, f.q, f.dq);
+    hipLaunchKernelGGL(k_ghost_dq, dim3(nblk(m.nBFace, kBlock)), dim3(kBlock), 0, s, m, k, f.q, f.dq,
+                       f.bwdFlow ? f.dqAlt : f.dq);
 }
 
 void launch_update(const DevMesh &m, const Consts &k, DevFlow &f, bool advance, hipStream_t s)

@@ -795,7 +795,7 @@ __global__ void __launch_bounds__(kBlock) k_sa_ghost_dq(DevMesh M, double *__res
     const bool copy = bc == kBC_FAR || bc == kBC_SYMM || bc == kBC_INFLOW || bc == kBC_OUTFLOW;
     const double v = copy ? dq[M.fle[f]] : 0.0;
     dq[M.nCell + f] = v;
-    rows[(size_t)(M.nCell + f) * kRow + 5] = v;
+    rows[((size_t)(kPlanes - 1) * M.nTotal + M.nCell + f) * 2 + 1] = v;  // the sixth value of the ghost's dq row
 }
 
 __global__ void __launch_bounds__(kBlock) k_sa_update(DevMesh M, double *__restrict__ nut,
@@ -904,7 +904,8 @@ void launch_sa_sweep_init(const DevMesh &m, DevFlow &f, hipStream_t s)
 void launch_sa_ghost_dq(const DevMesh &m, DevFlow &f, hipStream_t s)
 {
     if (m.nBFace > 0)
-        hipLaunchKernelGGL(k_sa_ghost_dq, dim3(nblk(m.nBFace, kBlock)), dim3(kBlock), 0, s, m, f.dqT, f.dq);
+        hipLaunchKernelGGL(k_sa_ghost_dq, dim3(nblk(m.nBFace, kBlock)), dim3(kBlock), 0, s, m, f.dqT,
+                           f.bwdFlow ? f.dqAlt : f.dq);
 }
 
 void launch_sa_update(const DevMesh &m, DevFlow &f, hipStream_t s)
@@ -936,10 +937,10 @@ void launch_sa_lusgs(const DevMesh &m, const Consts &k, DevFlow &f, const Levels
     log->done = 0;
     for (int it = 0; it < k.nSweeps; ++it) {
         sa_sweep_dispatch(m, f, fwd, true, s);
-        launch_sweep_change(f.dqT, 1, 0, 1, m.nCell, f.dqTPrev, f.sweepParts, f.sweepNorm, s);
+        launch_sweep_change(f.dqT, m.nCell, 1, m.nCell, f.dqTPrev, f.sweepParts, f.sweepNorm, s);
         launch_sa_ghost_dq(m, f, s);
         sa_sweep_dispatch(m, f, bwd, true, s);
-        launch_sweep_change(f.dqT, 1, 0, 1, m.nCell, f.dqTPrev, f.sweepParts, f.sweepNorm + 1, s);
+        launch_sweep_change(f.dqT, m.nCell, 1, m.nCell, f.dqTPrev, f.sweepParts, f.sweepNorm + 1, s);
         (void)hipMemcpyAsync(log->host, f.sweepNorm, 2 * sizeof(double), hipMemcpyDeviceToHost, s);
         if (hipStreamSynchronize(s) != hipSuccess) break;  // reported by the caller's launch check
         const double sn = log->host[0] + log->host[1];

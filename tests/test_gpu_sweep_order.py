@@ -46,3 +46,67 @@ def test_sweep_level_storage_equals_mesh_storage(name):
     a, b = run(mesh, 4, storage_order=0), run(mesh, 4, storage_order=1)
     for k in a:
         assert np.array_equal(a[k], b[k]), (name, k)
+
+
+@pytest.mark.parametrize("form", [0, 2, 3])
+@pytest.mark.parametrize("name", sorted(shapes()))
+def test_dataflow_sweep_at_chunk_edges_equals_level_form(name, form):
+    mesh = shapes()[name]()
+    a, b = run(mesh, 4, sweep_form=form), run(mesh, 4, sweep_form=1)
+    for k in a:
+        assert np.array_equal(a[k], b[k]), (name, k)
+
+
+def wide_cell_mesh(wide_first):
+    """Two columns of 3x3 unit cells' worth of space: one 1x3x3 polyhedron
+    whose inner side is nine faces, and nine unit hexahedra.  Numbered first, the polyhedron
+    has nine higher neighbours (a backward sweep too wide for the dataflow
+    form, a forward one that is not); numbered last, nine lower ones."""
+    xs = [(i, j, k) for i in range(3) for j in range(4) for k in range(4)]
+    node = {p: n for n, p in enumerate(xs)}
+    quad = lambda pts: [node[p] for p in pts]
+    big, small = (0, 1) if wide_first else (9, 0)
+    cell = lambda j, k: small + 3 * k + j
+    bnd, inner = [], []
+    ring = [(0, j, 0) for j in range(4)] + [(0, 3, k) for k in range(1, 4)] + [(0, j, 3) for j in (2, 1, 0)] + \
+           [(0, 0, k) for k in (2, 1)]
+    bnd.append((quad(ring)[::-1], big))
+    for j in range(3):  # the polyhedron's own y and z sides
+        bnd.append((quad([(0, j, 0), (1, j, 0), (1, j + 1, 0), (0, j + 1, 0)])[::-1], big))
+        bnd.append((quad([(0, j, 3), (1, j, 3), (1, j + 1, 3), (0, j + 1, 3)]), big))
+        bnd.append((quad([(0, 0, j), (0, 0, j + 1), (1, 0, j + 1), (1, 0, j)])[::-1], big))
+        bnd.append((quad([(0, 3, j), (0, 3, j + 1), (1, 3, j + 1), (1, 3, j)]), big))
+    for k in range(3):
+        for j in range(3):
+            x = lambda i: quad([(i, j, k), (i, j + 1, k), (i, j + 1, k + 1), (i, j, k + 1)])
+            a, b = (big, cell(j, k)) if wide_first else (cell(j, k), big)
+            inner.append((x(1) if wide_first else x(1)[::-1], a, b))
+            bnd.append((x(2), cell(j, k)))
+            y = lambda jj: quad([(1, jj, k), (1, jj, k + 1), (2, jj, k + 1), (2, jj, k)])
+            z = lambda kk: quad([(1, j, kk), (2, j, kk), (2, j + 1, kk), (1, j + 1, kk)])
+            if j == 0: bnd.append((y(0)[::-1], cell(j, k)))
+            if j == 2: bnd.append((y(3), cell(j, k)))
+            else: inner.append((y(j + 1), cell(j, k), cell(j + 1, k)))
+            if k == 0: bnd.append((z(0)[::-1], cell(j, k)))
+            if k == 2: bnd.append((z(3), cell(j, k)))
+            else: inner.append((z(k + 1), cell(j, k), cell(j, k + 1)))
+    nodes = {big: sorted({n for f, *cs in bnd + inner if big in cs for n in f})}
+    for j in range(3):
+        for k in range(3):
+            nodes[cell(j, k)] = [node[(i, j + a, k + b)] for i in (1, 2) for a in (0, 1) for b in (0, 1)]
+    faces = [f for f, *_ in bnd + inner]
+    return pa.Mesh.from_arrays(
+        *np.array(xs, float).T, np.cumsum([0] + [len(f) for f in faces]), np.concatenate(faces),
+        [c for _, c in bnd] + [a for _, a, _ in inner], [10 + n for n in range(len(bnd))] + [b for *_, b in inner],
+        len(bnd), [pa.BC["farfield"]] * len(bnd), np.cumsum([0] + [len(nodes[c]) for c in range(10)]),
+        np.concatenate([nodes[c] for c in range(10)]))
+
+
+@pytest.mark.parametrize("wide_first", [True, False])
+def test_one_direction_in_dataflow_form_the_other_by_level(wide_first):
+    mesh = wide_cell_mesh(wide_first)
+    met = mesh.metrics()
+    assert met["vol"][:10].min() > 0 and abs(met["vol"][:10].sum() - 18.0) < 1e-12
+    a, b = run(mesh, 5, sweep_form=0), run(mesh, 5, sweep_form=1)
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
