@@ -1,6 +1,7 @@
 // phl_mpnn.hip -- the warm-start message-passing network on gfx950: forward,
 // backward and Adam, hand-written, FP32 with the dense layers on MFMA
-// (v_mfma_f32_32x32x2_f32).  The network (no reference counterpart):
+// (v_mfma_f32_32x32x16_bf16 on exact three-way splits of the FP32 operands).
+// The network (no reference counterpart):
 //
 //     h0 = relu(X W0 + b0)                     X [N, 8] cell features
 //     l = 1..L:  m = mean_{j in N(i)} h_j       (face neighbours)
@@ -22,267 +23,309 @@ namespace {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int H = kHidden;    // 128
-constexpr int KC = 32;        // K chunk staged in LDS
 constexpr int TR = 128;       // rows per workgroup tile
 constexpr int kThreads = 256; // 4 waves
 constexpr int kRowChunk = 2048;  // rows per partial of a weight gradient
 constexpr int kMaxDeg = 8;       // neighbour lists up to this width take the batched-load path
 
-// D(32x32) += A(32x2) * B(2x32).  Lane l holds A[l % 32][l / 32] and
-// B[l / 32][l % 32]; accumulator register r of lane l holds
+// The 32x32 accumulator tiles of MFMA: register r of lane l holds
 // D[(r % 4) + 4 * (l / 32) + 8 * (r / 4)][l % 32].
 __device__ __forceinline__ int acc_row(int r, int lane) { return (r & 3) + 4 * (lane >> 5) + 8 * (r >> 2); }
 
-// C[N, 128] = A1[N, K1] W1[K1, 128] (+ A2[N, 128] W2[128, 128]) + bias,
-// W given row-major [K, 128], or transposed ([128, K], TW) for the backward
-// products dZ W^T.  Epilogue: z = C stored to Z (if non-null); out = z
-// (mode 0), relu(z) (mode 1), Hres + relu(z) (mode 2) or Hres + z (mode 3).
-// One thread's share of a K chunk, as float4: A [TR][KC] and W [KC][H] are
-// 1024 float4 each, 4 per thread.  K is a multiple of 4 (kIn or kHidden), so
-// a float4 is either wholly inside K or wholly past it; rows and weight
-// offsets are multiples of 4 floats, so every float4 load is aligned.
-static_assert(kIn % 4 == 0 && H % 4 == 0, "float4 staging needs K % 4 == 0");
-constexpr int kVec = TR * KC / 4 / kThreads;  // 4
-static_assert(TR * KC == KC * H && kVec * 4 * kThreads == TR * KC, "A and W chunks have the same size");
-
-struct Chunk {
-    float4 a[kVec], w[kVec];
-};
-
-template <bool TW>
-__device__ __forceinline__ void load_chunk(Chunk &st, const float *__restrict__ A, const float *__restrict__ W,
-                                           int N, int K, int row0, int k0)
-{
-#pragma unroll
-    for (int i = 0; i < kVec; ++i) {
-        const int q = threadIdx.x + i * kThreads;
-        const int row = row0 + (q >> 3), k = k0 + 4 * (q & 7);  // A: row q/8, k 4(q%8)..+3
-        st.a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (row < N && k < K) st.a[i] = *(const float4 *)(A + (size_t)row * K + k);
-        st.w[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (TW) {  // W^T stored [H][K]: column q/8, k 4(q%8)..+3
-            if (k < K) st.w[i] = *(const float4 *)(W + (size_t)(q >> 3) * K + k);
-        } else {   // W stored [K][H]: k q/32, columns 4(q%32)..+3
-            const int kw = k0 + (q >> 5);
-            if (kw < K) st.w[i] = *(const float4 *)(W + (size_t)kw * H + 4 * (q & 31));
-        }
-    }
-}
-
-template <bool TW>
-__device__ __forceinline__ void store_chunk(const Chunk &st, float (*Al)[KC + 1], float (*Wl)[H + 4])
-{
-#pragma unroll
-    for (int i = 0; i < kVec; ++i) {
-        const int q = threadIdx.x + i * kThreads;
-        const int r = q >> 3, kk = 4 * (q & 7);
-        Al[r][kk] = st.a[i].x;
-        Al[r][kk + 1] = st.a[i].y;
-        Al[r][kk + 2] = st.a[i].z;
-        Al[r][kk + 3] = st.a[i].w;
-        if (TW) {
-            Wl[kk][r] = st.w[i].x;
-            Wl[kk + 1][r] = st.w[i].y;
-            Wl[kk + 2][r] = st.w[i].z;
-            Wl[kk + 3][r] = st.w[i].w;
-        } else {
-            const int kw = q >> 5, c = 4 * (q & 31);
-            Wl[kw][c] = st.w[i].x;
-            Wl[kw][c + 1] = st.w[i].y;
-            Wl[kw][c + 2] = st.w[i].z;
-            Wl[kw][c + 3] = st.w[i].w;
-        }
-    }
-}
-
-// The next chunk's loads are issued before the MFMAs of the current one and
-// land in registers while they run; the LDS tiles are rewritten between two
-// barriers.
-template <bool TW>
-__device__ __forceinline__ void accumulate(f32x16 (&acc)[4], float (*Al)[KC + 1], float (*Wl)[H + 4],
-                                           const float *__restrict__ A, const float *__restrict__ W, int N, int K,
-                                           int row0)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    Chunk st;
-    load_chunk<TW>(st, A, W, N, K, row0, 0);
-    for (int k0 = 0; k0 < K; k0 += KC) {
-        __syncthreads();
-        store_chunk<TW>(st, Al, Wl);
-        __syncthreads();
-        load_chunk<TW>(st, A, W, N, K, row0, k0 + KC);  // past K: zeros, no loads
-        const int kmax = (K - k0 < KC) ? (K - k0) : KC;
-        for (int kk = 0; kk < kmax; kk += 2) {
-            const float a = Al[wave * 32 + (lane & 31)][kk + (lane >> 5)];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const float w = Wl[kk + (lane >> 5)][b * 32 + (lane & 31)];
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, w, acc[b], 0, 0, 0);
-            }
-        }
-    }
-}
-
-template <bool TW>
-__global__ void __launch_bounds__(kThreads, 2) k_dense(const float *__restrict__ A1, const float *__restrict__ W1, int K1,
-                                                    const float *__restrict__ A2, const float *__restrict__ W2,
-                                                    const float *__restrict__ bias, int N, int mode,
-                                                    const float *__restrict__ Hres, float *__restrict__ Z,
+// Input layer: z = X W0 + b0, out = relu(z); Z may be null.  Eight products
+// per output, so the 512-byte rows written bound it: a thread keeps its four
+// columns of W0 and walks kInRows rows.
+constexpr int kInRows = 16;
+__global__ void __launch_bounds__(kThreads) k_input(const float *__restrict__ X, const float *__restrict__ W0,
+                                                    const float *__restrict__ b0, int N, float *__restrict__ Z,
                                                     float *__restrict__ out)
 {
-    __shared__ float Al[TR][KC + 1];
-    __shared__ float Wl[KC][H + 4];
-    const int row0 = blockIdx.x * TR;
-    f32x16 acc[4];
+    static_assert(kIn == 8 && H == 128, "k_input's thread layout");
+    const int c = 4 * ((int)threadIdx.x & 31);
+    float4 w[kIn];
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int k = 0; k < kIn; ++k) w[k] = *(const float4 *)(W0 + k * H + c);
+    const float4 b = *(const float4 *)(b0 + c);
+    const int r0 = blockIdx.x * (8 * kInRows) + ((int)threadIdx.x >> 5);
+#pragma unroll 4
+    for (int i = 0; i < kInRows; ++i) {
+        const int row = r0 + 8 * i;
+        if (row >= N) return;
+        const float4 x0 = *(const float4 *)(X + (size_t)row * kIn), x1 = *(const float4 *)(X + (size_t)row * kIn + 4);
+        const float x[kIn] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
-    accumulate<TW>(acc, Al, Wl, A1, W1, N, K1, row0);
-    if (A2) accumulate<TW>(acc, Al, Wl, A2, W2, N, H, row0);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = row0 + wave * 32 + acc_row(r, lane);
-            const int col = b * 32 + (lane & 31);
-            if (row >= N) continue;
-            const size_t o = (size_t)row * H + col;
-            const float z = acc[b][r] + (bias ? bias[col] : 0.f);
-            if (Z) Z[o] = z;
-            const float rz = z > 0.f ? z : 0.f;
-            out[o] = mode == 0 ? z : (mode == 1 ? rz : (mode == 2 ? Hres[o] + rz : Hres[o] + z));
+        for (int k = 0; k < kIn; ++k) {
+            z.x = fmaf(x[k], w[k].x, z.x);
+            z.y = fmaf(x[k], w[k].y, z.y);
+            z.z = fmaf(x[k], w[k].z, z.z);
+            z.w = fmaf(x[k], w[k].w, z.w);
         }
+        z.x += b.x;
+        z.y += b.y;
+        z.z += b.z;
+        z.w += b.w;
+        const size_t o = (size_t)row * H + c;
+        if (Z) *(float4 *)(Z + o) = z;
+        *(float4 *)(out + o) = make_float4(z.x > 0.f ? z.x : 0.f, z.y > 0.f ? z.y : 0.f, z.z > 0.f ? z.z : 0.f,
+                                           z.w > 0.f ? z.w : 0.f);
+    }
 }
 
-// ---- BF16 form of the hidden layers' products (inference) ----
-// z = h A + m B + c with h, m and the weights rounded to BF16 (round to
-// nearest even, v_cvt_pk_bf16_f32) and FP32 accumulation on
-// v_mfma_f32_32x32x16_bf16; h' = h + relu(z) in FP32.  The weights come
-// transposed ([128 columns][128 k], BF16) from k_weights_bf16, so that each
-// lane's eight consecutive k of a B operand are one 16-byte LDS read, as
-// are the eight k of its A operand.  Lane l supplies A[l % 32][8 (l / 32) ..
-// + 7] and B[8 (l / 32) .. + 7][l % 32] of a K = 16 step; the accumulator
-// layout is the one of the FP32 instruction (acc_row).
+// ---- products on BF16 matrix cores ----
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// x as NP BF16 pieces.  NP 1: x rounded to nearest even.  NP 3: the exact
+// sum of three pieces (8 significant bits each, 24 in all): piece 0 is x
+// rounded, piece 1 the remainder rounded, piece 2 what is left.  That holds
+// below kSplitTop (magnitude bits), from which on x rounds to infinity.
+constexpr unsigned kSplitTop = 0x7f7f8000u;
+__device__ __forceinline__ bool splits(float x) { return (__float_as_uint(x) & 0x7fffffffu) < kSplitTop; }
+template <int NP>
+__device__ __forceinline__ void split(float x, __bf16 *p)
+{
+    p[0] = (__bf16)x;
+    if constexpr (NP == 3) {
+        const float r = x - (float)p[0];
+        p[1] = (__bf16)r;
+        p[2] = (__bf16)(r - (float)p[1]);
+    }
+}
+
+// The products of two three-piece operands that are kept beside the leading
+// one: piece kTermA against piece kTermB.  The dropped terms are below 2^-25 of
+// the product, half the rounding of an FP32 product.
+constexpr int kTerms = 5, kTermA[kTerms] = {2, 0, 1, 1, 0}, kTermB[kTerms] = {0, 2, 1, 0, 1};
+
+// out[N, 128] = A1[N, 128] W1 (+ A2[N, 128] W2) + bias, W1 and W2 as NP
+// pieces from k_split_weights; A split while it is staged.  Epilogue: z =
+// product + bias stored to Z (if non-null); out = z (mode 0), Hres + relu(z)
+// (mode 2) or Hres + z (mode 3).
+//
+// A workgroup makes 128 rows x 128 columns, each of its four waves 64 x 64 in
+// 2 x 2 accumulator tiles.  A runs through two LDS buffers of KB columns,
+// the loads one chunk ahead of the stores and the stores one ahead of the
+// products.  Lane l supplies A[l % 32][8 (l / 32) .. + 7] and
+// B[8 (l / 32) .. + 7][l % 32] of a K = 16 step: A in one 16-byte LDS read per
+// piece; the weights lie in memory as such operands, 1 KB per wave and piece,
+// and come from the L2 caches straight into registers, a step ahead.
+//
+// NP 3 replaces v_mfma_f32_32x32x2_f32 (157 TFLOP/s): six BF16 products of
+// 16 k take 192 cycles against 512.  Its error against 64 bits is no larger:
+// network output 2.5e-7 against 2.9e-7 (200,704 rows), gradients 2.4e-7 both
+// at 315 rows and 8e-7 against 1.0e-6 at 123,240; with all six products in one
+// accumulator the gradients at 315 rows were 4% off more.  A hidden layer of
+// 200,704 rows takes 131 us instead of 262 (66 us are the bytes alone), bound
+// by the latency of a workgroup's eight chunks at two workgroups per CU.  NP 1 (inference) is bound by its 1,536 bytes of
+// activations per row: 621,818 rows in 224 us instead of 351, 4.3 TB/s.
+//
+// A value that does not split (kSplitTop; infinities and NaN among them), in
+// the rows or in the weights (`bad`, one int per workgroup of
+// k_split_weights), makes its tile be summed again value by value in FP32.
 constexpr int KB = 32;       // K chunk staged in LDS
-constexpr int KBP = KB + 8;  // LDS row length: 80-byte rows keep every 16-byte read aligned
-static_assert(kVec * 4 * kThreads == TR * KB && 2 * 8 * kThreads == H * KB, "BF16 chunk shares");
+constexpr int KBP = KB + 8;  // LDS row length: 80-byte rows keep every 16-byte read aligned and conflict-free
+constexpr int kVec = TR * KB / 4 / kThreads;  // float4 of A per thread and chunk (4)
+constexpr int kSteps = KB / 16;               // K steps per chunk
+static_assert(kVec * 4 * kThreads == TR * KB && H == TR, "chunk shares");
+static_assert(kBadFlags == H * H / kThreads && kBadFlags == 64, "one flag per workgroup and per lane");
 
-struct ChunkB {
-    float4 a[kVec];  // A [TR][KB]: row q/8, k 4(q%8)..+3
-    uint4 w[2];      // W^T [H][KB]: column q/4, k 8(q%4)..+7
-};
+// Element (k, column) of a piece of a weight matrix in operand order:
+// [K step of 16][32 columns][lane][8].
+__device__ __forceinline__ int weight_at(int k, int col)
+{
+    return (((k >> 4) * (H / 32) + (col >> 5)) * 64 + ((k >> 3) & 1) * 32 + (col & 31)) * 8 + (k & 7);
+}
 
-__device__ __forceinline__ void load_chunk_bf16(ChunkB &st, const float *__restrict__ A,
-                                                const __bf16 *__restrict__ Wt, int N, int row0, int k0)
+__device__ __forceinline__ void load_rows(float4 (&st)[kVec], const float *__restrict__ A, int N, int row0, int k0)
 {
 #pragma unroll
-    for (int i = 0; i < kVec; ++i) {
+    for (int i = 0; i < kVec; ++i) {  // A [TR][KB]: row q/8, k 4(q%8)..+3; rows past N repeat the last
         const int q = threadIdx.x + i * kThreads;
-        const int row = row0 + (q >> 3), k = k0 + 4 * (q & 7);
-        st.a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (row < N && k < H) st.a[i] = *(const float4 *)(A + (size_t)row * H + k);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int q = threadIdx.x + i * kThreads;
-        const int k = k0 + 8 * (q & 3);
-        st.w[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (k < H) st.w[i] = *(const uint4 *)(Wt + (size_t)(q >> 2) * H + k);
+        st[i] = *(const float4 *)(A + (size_t)min(row0 + (q >> 3), N - 1) * H + k0 + 4 * (q & 7));
     }
 }
 
-__device__ __forceinline__ void store_chunk_bf16(const ChunkB &st, __bf16 (*Al)[KBP], __bf16 (*Wl)[KBP])
+// Also the largest magnitude (as bits) of the values stored.
+template <int NP>
+__device__ __forceinline__ unsigned store_rows(const float4 (&st)[kVec], __bf16 (*Al)[TR][KBP])
 {
+    unsigned top = 0;
 #pragma unroll
     for (int i = 0; i < kVec; ++i) {
         const int q = threadIdx.x + i * kThreads;
-        bf16x4 v;
-        v[0] = (__bf16)st.a[i].x;
-        v[1] = (__bf16)st.a[i].y;
-        v[2] = (__bf16)st.a[i].z;
-        v[3] = (__bf16)st.a[i].w;
-        *(bf16x4 *)&Al[q >> 3][4 * (q & 7)] = v;
-    }
+        const float x[4] = {st[i].x, st[i].y, st[i].z, st[i].w};
+        bf16x4 v[NP];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int q = threadIdx.x + i * kThreads;
-        *(uint4 *)&Wl[q >> 2][8 * (q & 3)] = st.w[i];
+        for (int e = 0; e < 4; ++e) {
+            __bf16 pc[NP];
+            split<NP>(x[e], pc);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) v[p][e] = pc[p];
+            if constexpr (NP == 3) top = max(top, __float_as_uint(x[e]) & 0x7fffffffu);
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) *(bf16x4 *)&Al[p][q >> 3][4 * (q & 7)] = v[p];
     }
+    return top;
 }
 
-__device__ __forceinline__ void accumulate_bf16(f32x16 (&acc)[4], __bf16 (*Al)[KBP], __bf16 (*Wl)[KBP],
-                                                const float *__restrict__ A, const __bf16 *__restrict__ Wt, int N,
-                                                int row0)
+// The wave's weight operands of K step `step`.
+template <int NP>
+__device__ __forceinline__ void load_weights(bf16x8 (&w)[NP][2], const __bf16 *__restrict__ W, int step, int wc,
+                                             int lane)
 {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            w[p][j] = *(const bf16x8 *)(W + (size_t)p * H * H + ((step * (H / 32) + (wc >> 5) + j) * 64 + lane) * 8);
+}
+
+// One value of A W summed in FP32.
+__device__ float dot_fp32(const Product &p, bool transpose, int row, int col, float s)
+{
+    for (int k = 0; k < H; ++k)
+        s = fmaf(p.A[(size_t)row * H + k], p.W32[transpose ? col * H + k : k * H + col], s);
+    return s;
+}
+
+template <int NP>
+__global__ void __launch_bounds__(kThreads, 2) k_dense(Product P1, Product P2, bool transpose,
+                                                       const float *__restrict__ bias, int N, int mode,
+                                                       const float *__restrict__ Hres, float *__restrict__ Z,
+                                                       float *__restrict__ out)
+{
+    const float *__restrict__ A1 = P1.A, *__restrict__ A2 = P2.A;
+    const __bf16 *__restrict__ W1 = P1.W, *__restrict__ W2 = P2.W;
+    __shared__ __attribute__((aligned(16))) __bf16 Al[2][NP][TR][KBP];
+    const int row0 = blockIdx.x * TR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    ChunkB st;
-    load_chunk_bf16(st, A, Wt, N, row0, 0);
-    for (int k0 = 0; k0 < H; k0 += KB) {
-        __syncthreads();
-        store_chunk_bf16(st, Al, Wl);
-        __syncthreads();
-        load_chunk_bf16(st, A, Wt, N, row0, k0 + KB);  // past K: zeros, no loads
+    const int wr = 64 * (wave >> 1), wc = 64 * (wave & 1);  // the wave's rows and columns
+    f32x16 acc[2][2];
 #pragma unroll
-        for (int ks = 0; ks < KB; ks += 16) {
-            const bf16x8 a = *(const bf16x8 *)&Al[wave * 32 + (lane & 31)][ks + 8 * (lane >> 5)];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const bf16x8 w = *(const bf16x8 *)&Wl[b * 32 + (lane & 31)][ks + 8 * (lane >> 5)];
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w, acc[b], 0, 0, 0);
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    constexpr int half = H / KB;  // chunks of one operand
+    const int chunks = A2 ? 2 * half : half;
+    int odd = 0;  // a value that does not split was met
+    if constexpr (NP == 3) odd = P1.bad[lane] | (A2 ? P2.bad[lane] : 0);
+    float4 st[kVec];
+    bf16x8 w[kSteps][NP][2];
+    load_rows(st, A1, N, row0, 0);
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) load_weights<NP>(w[ks], W1, ks, wc, lane);
+    odd |= store_rows<NP>(st, Al[0]) >= kSplitTop;
+    load_rows(st, A1, N, row0, KB);
+    __syncthreads();
+    for (int ch = 0; ch < chunks; ++ch) {
+        const int nc = ch + 1;
+        const __bf16 *Wn = nc >= half ? W2 : W1;
+#pragma unroll
+        for (int ks = 0; ks < kSteps; ++ks) {
+            const int k = 16 * ks + 8 * (lane >> 5), l = lane & 31;
+            bf16x8 a[NP][2];
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) a[p][i] = *(const bf16x8 *)&Al[ch & 1][p][wr + 32 * i + l][k];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if constexpr (NP == 3) {
+                        // the five small terms on their own, so that the sum takes one rounding for them
+                        f32x16 t;
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) t[r] = 0.f;
+#pragma unroll
+                        for (int q = 0; q < kTerms; ++q)
+                            t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kTermA[q]][i], w[ks][kTermB[q]][j], t, 0, 0,
+                                                                        0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], w[ks][0][j], acc[i][j], 0, 0, 0);
+                        acc[i][j] += t;
+                    } else {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], w[ks][0][j], acc[i][j], 0, 0, 0);
+                    }
+                }
+            // this step's weights of the next chunk
+            if (nc < chunks) load_weights<NP>(w[ks], Wn, (nc % half) * kSteps + ks, wc, lane);
+        }
+        if (nc < chunks) odd |= store_rows<NP>(st, Al[nc & 1]) >= kSplitTop;
+        if (ch + 2 < chunks) load_rows(st, ch + 2 >= half ? A2 : A1, N, row0, ((ch + 2) % half) * KB);
+        __syncthreads();
+    }
+    if (NP == 3 && __syncthreads_or(odd)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int row = row0 + wr + 32 * i + acc_row(r, lane), col = wc + 32 * j + (lane & 31);
+                    if (row >= N) continue;
+                    float v = dot_fp32(P1, transpose, row, col, 0.f);
+                    if (A2) v = dot_fp32(P2, transpose, row, col, v);
+                    acc[i][j][r] = v;
+                }
+    }
+    // one 32 x 32 tile at a time, its 16 residual loads in flight together
+    // (behind a branch per row each would wait for the one before it); rows
+    // past N are clamped for the loads and left out of the stores
+    const bool full = row0 + TR <= N;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int col = wc + 32 * j + (lane & 31);
+            const float bc = bias ? bias[col] : 0.f;
+            float h[16];
+            if (mode != 0) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    h[r] = Hres[(size_t)min(row0 + wr + 32 * i + acc_row(r, lane), N - 1) * H + col];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) h[r] = 0.f;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = row0 + wr + 32 * i + acc_row(r, lane);
+                const size_t o = (size_t)row * H + col;
+                const float z = acc[i][j][r] + bc;
+                const float v = mode == 0 ? z : (mode == 2 ? h[r] + (z > 0.f ? z : 0.f) : h[r] + z);
+                if (full || row < N) {
+                    if (Z) Z[o] = z;
+                    out[o] = v;
+                }
             }
         }
-    }
 }
 
-// out = H + relu(A1 W1 + A2 W2 + bias), A1 = h and A2 = m [N, 128] FP32, W1t,
-// W2t the layer's transposed BF16 weights.
-__global__ void __launch_bounds__(kThreads, 2) k_dense_bf16(const float *__restrict__ A1,
-                                                         const __bf16 *__restrict__ W1t,
-                                                         const float *__restrict__ A2,
-                                                         const __bf16 *__restrict__ W2t,
-                                                         const float *__restrict__ bias, int N,
-                                                         const float *__restrict__ Hres, float *__restrict__ out)
-{
-    __shared__ __attribute__((aligned(16))) __bf16 Al[TR][KBP];  // 16-byte reads and stores
-    __shared__ __attribute__((aligned(16))) __bf16 Wl[H][KBP];
-    const int row0 = blockIdx.x * TR;
-    f32x16 acc[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
-    accumulate_bf16(acc, Al, Wl, A1, W1t, N, row0);
-    accumulate_bf16(acc, Al, Wl, A2, W2t, N, row0);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = row0 + wave * 32 + acc_row(r, lane);
-            const int col = b * 32 + (lane & 31);
-            if (row >= N) continue;
-            const size_t o = (size_t)row * H + col;
-            const float z = acc[b][r] + bias[col];
-            out[o] = Hres[o] + (z > 0.f ? z : 0.f);
-        }
-}
-
-// The hidden layers' A_l and B_l [L][128 k][128 columns] FP32 to BF16,
-// transposed: out [L][2][128 columns][128 k] (A_l, then B_l).
-__global__ void __launch_bounds__(kThreads) k_weights_bf16(const float *__restrict__ A, const float *__restrict__ B,
-                                                           int L, __bf16 *__restrict__ out)
+// The hidden layers' A_l and B_l [L][128][128] FP32 as NP BF16 pieces in
+// operand order, out [L][2][NP][128 * 128] (A_l, then B_l): as they are for the
+// forward products h A, m B (k the row), or transposed for the backward
+// products dz A^T, dz B^T (k the column).
+template <int NP>
+__global__ void __launch_bounds__(kThreads) k_split_weights(const float *__restrict__ A, const float *__restrict__ B,
+                                                            int L, bool transpose, __bf16 *__restrict__ out,
+                                                            int *__restrict__ bad)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t HH = (size_t)H * H;
-    if (i >= (size_t)L * 2 * HH) return;
-    const size_t l = i / (2 * HH), r = i % (2 * HH);
-    const int which = (int)(r / HH), col = (int)((r % HH) / H), k = (int)(r % H);
-    const float *src = which ? B : A;
-    out[i] = (__bf16)src[l * HH + (size_t)k * H + col];
+    static_assert(H * H % kThreads == 0, "the grid covers whole matrices");
+    const size_t lw = i / HH, r = i % HH;
+    const int u = (int)(r / H), v = (int)(r % H);  // W[u][v] of the layer's matrix
+    const float w = (((lw & 1) ? B : A) + (lw >> 1) * HH)[r];
+    __bf16 p[NP];
+    split<NP>(w, p);
+#pragma unroll
+    for (int q = 0; q < NP; ++q) out[(lw * NP + q) * HH + (transpose ? weight_at(v, u) : weight_at(u, v))] = p[q];
+    const int any = __syncthreads_or(!splits(w));
+    if (threadIdx.x == 0) bad[blockIdx.x] = any;
 }
 
 constexpr int kPer = 32 * H / kThreads;  // elements of a 32-row slab staged per thread
@@ -563,27 +606,25 @@ inline int nb(size_t n, int b) { return (int)((n + b - 1) / b); }
 }  // namespace
 
 // ---------------------------------------------------------------- launchers
-void dense(const float *A1, const float *W1, int K1, const float *A2, const float *W2, const float *bias, int N,
-           int mode, const float *Hres, float *Z, float *out, bool transW, hipStream_t s)
+void input_layer(const float *X, const float *W0, const float *b0, int N, float *Z, float *out, hipStream_t s)
 {
-    if (transW)
-        hipLaunchKernelGGL(k_dense<true>, dim3(nb(N, TR)), dim3(kThreads), 0, s, A1, W1, K1, A2, W2, bias, N, mode,
-                           Hres, Z, out);
-    else
-        hipLaunchKernelGGL(k_dense<false>, dim3(nb(N, TR)), dim3(kThreads), 0, s, A1, W1, K1, A2, W2, bias, N, mode,
-                           Hres, Z, out);
+    hipLaunchKernelGGL(k_input, dim3(nb(N, 8 * kInRows)), dim3(kThreads), 0, s, X, W0, b0, N, Z, out);
 }
 
-void weights_bf16(const float *A, const float *B, int L, __bf16 *out, hipStream_t s)
+void split_weights(const float *A, const float *B, int L, int pieces, bool transpose, __bf16 *out, int *bad,
+                   hipStream_t s)
 {
-    const size_t n = (size_t)L * 2 * H * H;
-    hipLaunchKernelGGL(k_weights_bf16, dim3((unsigned)nb(n, kThreads)), dim3(kThreads), 0, s, A, B, L, out);
+    const dim3 g((unsigned)nb((size_t)L * 2 * H * H, kThreads));
+    if (pieces == 3) hipLaunchKernelGGL(k_split_weights<3>, g, dim3(kThreads), 0, s, A, B, L, transpose, out, bad);
+    else hipLaunchKernelGGL(k_split_weights<1>, g, dim3(kThreads), 0, s, A, B, L, transpose, out, bad);
 }
 
-void dense_bf16(const float *h, const __bf16 *At, const float *m, const __bf16 *Bt, const float *bias, int N,
-                float *out, hipStream_t s)
+void dense(const Product &p1, const Product &p2, bool transpose, const float *bias, int N, int mode,
+           const float *Hres, float *Z, float *out, int pieces, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_dense_bf16, dim3(nb(N, TR)), dim3(kThreads), 0, s, h, At, m, Bt, bias, N, h, out);
+    const dim3 g(nb(N, TR)), b(kThreads);
+    if (pieces == 3) hipLaunchKernelGGL(k_dense<3>, g, b, 0, s, p1, p2, transpose, bias, N, mode, Hres, Z, out);
+    else hipLaunchKernelGGL(k_dense<1>, g, b, 0, s, p1, p2, transpose, bias, N, mode, Hres, Z, out);
 }
 
 int grad_parts(int N) { return nb(N, kRowChunk); }

@@ -36,7 +36,9 @@ struct phl_mpnn {
     std::vector<void *> act;  // activation allocations (re-made per graph)
     // BF16 inference form of the hidden layers (phl_mpnn_set_forward_precision)
     int fwdBF16 = 0;
-    __bf16 *wt16 = nullptr;  // [L][2][128][128] transposed BF16 A_l, B_l
+    // the hidden layers' A_l, B_l as BF16 pieces (split_weights): up to three each
+    __bf16 *wt16 = nullptr;  // [L][2][3][128][128]
+    int *wtBad = nullptr;    // [L][2][kBadFlags] parts that are not finite
 };
 
 namespace {
@@ -99,39 +101,35 @@ phl_status alloc_activations(phl_mpnn *n)
     return PHL_OK;
 }
 
-void forward(phl_mpnn *n)
+// Rows A times A_l (which 0) or B_l (1) of the last split_weights.
+phl::nn::Product hidden_product(const phl_mpnn *n, const float *A, int l, int which, int pieces)
 {
-    using namespace phl::nn;
-    hipStream_t s = n->stream;
-    const int N = n->N;
-    const size_t NH = (size_t)N * kHidden, HH = (size_t)kHidden * kHidden;
-    dense(n->X, n->p + n->oW0, kIn, nullptr, nullptr, n->p + n->ob0, N, 1, nullptr, n->z0, n->hs, false, s);
-    for (int l = 0; l < n->L; ++l) {
-        float *h = n->hs + NH * l, *hn = n->hs + NH * (l + 1);
-        neighbour_mean(n->nbr, n->W, N, n->invDeg, h, n->ms + NH * l, s);
-        dense(h, n->p + n->oA + HH * l, kHidden, n->ms + NH * l, n->p + n->oB + HH * l, n->p + n->oc + kHidden * l, N,
-              2, h, n->zs + NH * l, hn, false, s);
-    }
-    out_layer(n->hs + NH * n->L, n->p + n->oWo, n->p + n->obo, N, n->y, s);
+    const size_t HH = (size_t)kHidden * kHidden, lw = 2 * (size_t)l + which;
+    return {A, n->wt16 + HH * pieces * lw, n->wtBad + phl::nn::kBadFlags * lw,
+            n->p + (which ? n->oB : n->oA) + HH * l};
 }
 
-// The inference pass with the hidden layers' products in BF16: the weights
-// are converted once per call; z is not kept (no backward pass follows).
-void forward_bf16(phl_mpnn *n)
+// The network on the current features.  For a backward pass (`keep`) every
+// layer's h, m and z stay in hs, ms and zs; an inference pass alternates
+// between two rows of hs and keeps no m or z, so that a layer's input is
+// still in cache when it is read.  pieces: 3 (FP32 products) or 1 (BF16).
+void forward(phl_mpnn *n, bool keep, int pieces)
 {
     using namespace phl::nn;
     hipStream_t s = n->stream;
     const int N = n->N;
-    const size_t NH = (size_t)N * kHidden, HH = (size_t)kHidden * kHidden;
-    weights_bf16(n->p + n->oA, n->p + n->oB, n->L, n->wt16, s);
-    dense(n->X, n->p + n->oW0, kIn, nullptr, nullptr, n->p + n->ob0, N, 1, nullptr, n->z0, n->hs, false, s);
+    const size_t NH = (size_t)N * kHidden;
+    split_weights(n->p + n->oA, n->p + n->oB, n->L, pieces, false, n->wt16, n->wtBad, s);
+    input_layer(n->X, n->p + n->oW0, n->p + n->ob0, N, keep ? n->z0 : nullptr, n->hs, s);
+    float *h = n->hs;
     for (int l = 0; l < n->L; ++l) {
-        float *h = n->hs + NH * l, *hn = n->hs + NH * (l + 1);
-        neighbour_mean(n->nbr, n->W, N, n->invDeg, h, n->ms + NH * l, s);
-        dense_bf16(h, n->wt16 + 2 * HH * l, n->ms + NH * l, n->wt16 + 2 * HH * l + HH, n->p + n->oc + kHidden * l, N,
-                   hn, s);
+        float *hn = n->hs + NH * (keep ? l + 1 : (l + 1) % 2), *m = n->ms + (keep ? NH * l : 0);
+        neighbour_mean(n->nbr, n->W, N, n->invDeg, h, m, s);
+        dense(hidden_product(n, h, l, 0, pieces), hidden_product(n, m, l, 1, pieces), false, n->p + n->oc + kHidden * l,
+              N, 2, h, keep ? n->zs + NH * l : nullptr, hn, pieces, s);
+        h = hn;
     }
-    out_layer(n->hs + NH * n->L, n->p + n->oWo, n->p + n->obo, N, n->y, s);
+    out_layer(h, n->p + n->oWo, n->p + n->obo, N, n->y, s);
 }
 
 // gradient of the loss into n->g (forward must have run; dy holds dL/dy)
@@ -144,15 +142,16 @@ void backward(phl_mpnn *n)
     small_grad(n->hs + NH * n->L, kHidden, n->dy, kOut, N, n->part, n->g + n->oWo, s);
     small_grad(nullptr, 1, n->dy, kOut, N, n->part, n->g + n->obo, s);
     out_layer_back(n->dy, n->p + n->oWo, N, n->dh, s);
+    split_weights(n->p + n->oA, n->p + n->oB, n->L, 3, true, n->wt16, n->wtBad, s);
     for (int l = n->L - 1; l >= 0; --l) {
         relu_back(n->dh, n->zs + NH * l, NH, n->dz, s);
         wgrad(n->hs + NH * l, n->dz, N, n->part, n->g + n->oA + HH * l, s);
         wgrad(n->ms + NH * l, n->dz, N, n->part, n->g + n->oB + HH * l, s);
         small_grad(nullptr, 1, n->dz, kHidden, N, n->part, n->g + n->oc + kHidden * l, s);
         // dm = dz B^T;  dh' = dh + dz A^T + (mean)^T dm
-        dense(n->dz, n->p + n->oB + HH * l, kHidden, nullptr, nullptr, nullptr, N, 0, nullptr, nullptr, n->dm, true,
-              s);
-        dense(n->dz, n->p + n->oA + HH * l, kHidden, nullptr, nullptr, nullptr, N, 3, n->dh, nullptr, n->dh2, true, s);
+        const Product none{};
+        dense(hidden_product(n, n->dz, l, 1, 3), none, true, nullptr, N, 0, nullptr, nullptr, n->dm, 3, s);
+        dense(hidden_product(n, n->dz, l, 0, 3), none, true, nullptr, N, 3, n->dh, nullptr, n->dh2, 3, s);
         neighbour_mean_transpose_add(n->nbr, n->W, N, n->invDeg, n->dm, n->dh2, s);
         std::swap(n->dh, n->dh2);
     }
@@ -188,7 +187,8 @@ phl_status phl_mpnn_create(int layers, unsigned seed, int device, phl_mpnn **out
     if (e == hipSuccess) e = hipMalloc(&n->g, bytes);
     if (e == hipSuccess) e = hipMalloc(&n->m, bytes);
     if (e == hipSuccess) e = hipMalloc(&n->v, bytes);
-    if (e == hipSuccess) e = hipMalloc(&n->wt16, sizeof(__bf16) * 2 * HH * layers);
+    if (e == hipSuccess) e = hipMalloc(&n->wtBad, sizeof(int) * 2 * phl::nn::kBadFlags * layers);
+    if (e == hipSuccess) e = hipMalloc(&n->wt16, sizeof(__bf16) * 2 * 3 * HH * layers);
     if (e != hipSuccess) {
         phl_mpnn_destroy(n);
         return fail(PHL_ERR_HIP, std::string("phl_mpnn_create: ") + hipGetErrorString(e));
@@ -219,6 +219,7 @@ void phl_mpnn_destroy(phl_mpnn *n)
     for (float *q : {n->p, n->g, n->m, n->v})
         if (q) hipFree(q);
     if (n->wt16) hipFree(n->wt16);
+    if (n->wtBad) hipFree(n->wtBad);
     if (n->nbr) hipFree(n->nbr);
     if (n->invDeg) hipFree(n->invDeg);
     if (n->stream) hipStreamDestroy(n->stream);
@@ -334,8 +335,7 @@ phl_status phl_mpnn_forward(phl_mpnn *n, float *Y)
 {
     if (!n || !Y || n->N == 0) return fail(PHL_ERR_ARG, "phl_mpnn_forward: no graph");
     HIPTRY(hipSetDevice(n->device));
-    if (n->fwdBF16) forward_bf16(n);
-    else forward(n);
+    forward(n, false, n->fwdBF16 ? 1 : 3);
     HIPTRY(hipGetLastError());
     HIPTRY(hipMemcpyAsync(Y, n->y, sizeof(float) * (size_t)n->N * kOut, hipMemcpyDeviceToHost, n->stream));
     HIPTRY(hipStreamSynchronize(n->stream));
@@ -353,7 +353,7 @@ phl_status phl_mpnn_gradient(phl_mpnn *n, double *lossOut, float *grad)
 {
     if (!n || n->N == 0) return fail(PHL_ERR_ARG, "phl_mpnn_gradient: no graph");
     HIPTRY(hipSetDevice(n->device));
-    forward(n);
+    forward(n, true, 3);
     phl::nn::loss(n->y, n->T, n->N * kOut, n->dy, n->lossPart, n->lossOut, n->stream);
     backward(n);
     HIPTRY(hipGetLastError());
@@ -370,7 +370,7 @@ phl_status phl_mpnn_train(phl_mpnn *n, int steps, float lr, double *lossHist)
     HIPTRY(hipSetDevice(n->device));
     std::vector<double> h(std::max(steps, 1));
     for (int i = 0; i < steps; ++i) {
-        forward(n);
+        forward(n, true, 3);
         phl::nn::loss(n->y, n->T, n->N * kOut, n->dy, n->lossPart, n->lossOut, n->stream);
         backward(n);
         ++n->step;

@@ -10,15 +10,28 @@ constexpr int kIn = 8;        // cell features
 constexpr int kHidden = 128;  // hidden width
 constexpr int kOut = 5;       // predicted state
 
-// out[N,128] = A1[N,K1] W1 (+ A2[N,128] W2) + bias, epilogue by mode (see the
-// kernel); transW takes W as [128,K] (the backward products dZ W^T).
-void dense(const float *A1, const float *W1, int K1, const float *A2, const float *W2, const float *bias, int N,
-           int mode, const float *Hres, float *Z, float *out, bool transW, hipStream_t s);
-// The BF16 inference form of a hidden layer: out = h + relu(h A + m B + c)
-// with BF16 products (FP32 accumulation); At, Bt from weights_bf16.
-void weights_bf16(const float *A, const float *B, int L, __bf16 *out, hipStream_t s);
-void dense_bf16(const float *h, const __bf16 *At, const float *m, const __bf16 *Bt, const float *bias, int N,
-                float *out, hipStream_t s);
+// out[N,128] = relu(X W0 + b0), before the relu also to Z (may be null).
+void input_layer(const float *X, const float *W0, const float *b0, int N, float *Z, float *out, hipStream_t s);
+// The hidden layers' A_l, B_l as BF16 pieces [L][2][pieces][128][128]: 3, whose
+// sum is the FP32 value, or 1, the value rounded to BF16; as they are for the
+// forward products, transposed for the backward ones.  bad [L][2][kBadFlags]:
+// whether part of a matrix does not split into pieces.
+constexpr int kBadFlags = 64;
+void split_weights(const float *A, const float *B, int L, int pieces, bool transpose, __bf16 *out, int *bad,
+                   hipStream_t s);
+// The operands of one product: rows A [N][128], the weights' pieces and flags
+// from split_weights, and the FP32 weights they were made of ([k][column], or
+// [column][k] when transposed).
+struct Product {
+    const float *A;
+    const __bf16 *W;
+    const int *bad;
+    const float *W32;
+};
+// out[N,128] = p1 (+ p2, if its A is not null) + bias, epilogue by mode (see
+// the kernel): FP32 products (3 pieces) or BF16 ones (1), FP32 accumulation.
+void dense(const Product &p1, const Product &p2, bool transpose, const float *bias, int N, int mode,
+           const float *Hres, float *Z, float *out, int pieces, hipStream_t s);
 int grad_parts(int N);
 // out[128,128] = A[N,128]^T D[N,128] (part: grad_parts(N) * 128 * 128 floats)
 void wgrad(const float *A, const float *D, int N, float *part, float *out, hipStream_t s);
