@@ -328,94 +328,214 @@ __global__ void __launch_bounds__(kThreads) k_split_weights(const float *__restr
     if (threadIdx.x == 0) bad[blockIdx.x] = any;
 }
 
-constexpr int kPer = 32 * H / kThreads;  // elements of a 32-row slab staged per thread
-
-// Partial of G[K, 128] = A[rows, K]^T D[rows, 128] over one chunk of
-// kRowChunk rows; K = 128.  Wave w owns G rows 32w..32w+31.
-__global__ void __launch_bounds__(kThreads) k_wgrad_part(const float *__restrict__ A, const float *__restrict__ D,
-                                                         int N, float *__restrict__ part)
+// ---- weight gradients ----
+// Sums over all rows, in two steps of fixed order: partials over chunks of
+// rows, then the partials (k_sum_parts).  A chunk is what gives about one
+// workgroup per CU, at most kRowChunk rows (the FP32 chain of a partial): with
+// 2,048 rows whatever N, 123,240 rows kept 61 of 256 CUs busy.
+constexpr int kSlab = 32;           // rows staged at a time
+constexpr int kSlabP = kSlab + 8;   // LDS row length, as KBP
+constexpr int kGradThreads = 512;   // waves 0-3: A^T D, waves 4-7: B^T D
+inline __host__ __device__ int grad_rows(int N)
 {
-    __shared__ float Al[32][H + 4];
-    __shared__ float Dl[32][H + 4];
+    const int r = ((N + 255) / 256 + kSlab - 1) / kSlab * kSlab;
+    return r < kRowChunk ? r : kRowChunk;
+}
+constexpr int kGradOut = 2 * H * H + H;  // A^T D, B^T D and the column sums of D
+
+// Partials of A^T D, B^T D [128, 128] and of the column sums of D over rows
+// r0 .. r0 + rows of A, B, D [N, 128], FP32 operands in three BF16 pieces as in
+// k_dense.  The products run along the rows, so a slab is staged transposed
+// ([feature][row], eight rows of a feature per 16-byte store) and a row of D
+// is read once for both products and the bias.  123,240 rows: 78 us, and 17
+// for the sum, for what took 420 (two products, FP32 MFMA) and 71 (the bias).
+__global__ void __launch_bounds__(kGradThreads, 2) k_wgrad_part(const float *__restrict__ A,
+                                                                const float *__restrict__ B,
+                                                                const float *__restrict__ D, int N, int rows,
+                                                                float *__restrict__ part)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 T[3][3][H][kSlabP];  // operand, piece, feature, row
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = blockIdx.x * kRowChunk;
-    f32x16 acc[4];
+    const int op = wave >> 2, wr = 64 * ((wave >> 1) & 1), wc = 64 * (wave & 1);
+    const int r0 = blockIdx.x * rows, r1 = min(r0 + rows, N);
+    const int f = threadIdx.x & (H - 1), g = threadIdx.x >> 7;  // staging: feature, rows 8g .. 8g + 7
+    f32x16 acc[2][2];
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
-    for (int s = 0; s < kRowChunk; s += 32) {
-        float va[kPer], vd[kPer];
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int e = threadIdx.x + i * kThreads;
-            const int row = r0 + s + e / H;
-            const bool in = row < N;
-            va[i] = in ? A[(size_t)row * H + e % H] : 0.f;
-            vd[i] = in ? D[(size_t)row * H + e % H] : 0.f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    float st[3][8], colSum = 0.f;
+    unsigned top = 0;
+    auto load = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int row = s + 8 * g + i;
+            const size_t o = (size_t)min(row, N - 1) * H + f;
+            const float a = A[o], b = B[o], d = D[o];
+            st[0][i] = row < r1 ? a : 0.f;
+            st[1][i] = row < r1 ? b : 0.f;
+            st[2][i] = row < r1 ? d : 0.f;
         }
+    };
+    load(r0);
+    for (int s = r0; s < r1; s += kSlab) {
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int e = threadIdx.x + i * kThreads;
-            Al[e / H][e % H] = va[i];
-            Dl[e / H][e % H] = vd[i];
-        }
-        __syncthreads();
-        for (int n = 0; n < 32; n += 2) {
-            const float a = Al[n + (lane >> 5)][wave * 32 + (lane & 31)];
+        for (int q = 0; q < 3; ++q) {
+            bf16x8 v[3];
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const float d = Dl[n + (lane >> 5)][b * 32 + (lane & 31)];
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, d, acc[b], 0, 0, 0);
+            for (int i = 0; i < 8; ++i) {
+                __bf16 p[3];
+                split<3>(st[q][i], p);
+                v[0][i] = p[0];
+                v[1][i] = p[1];
+                v[2][i] = p[2];
+                top = max(top, __float_as_uint(st[q][i]) & 0x7fffffffu);
             }
+#pragma unroll
+            for (int p = 0; p < 3; ++p) *(bf16x8 *)&T[q][p][f][8 * g] = v[p];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) colSum += st[2][i];
+        __syncthreads();
+        if (s + kSlab < r1) load(s + kSlab);
+#pragma unroll
+        for (int ks = 0; ks < kSlab; ks += 16) {
+            const int k = ks + 8 * (lane >> 5), l = lane & 31;
+            bf16x8 a[3][2], d[3][2];
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[p][i] = *(const bf16x8 *)&T[op][p][wr + 32 * i + l][k];
+                    d[p][i] = *(const bf16x8 *)&T[2][p][wc + 32 * i + l][k];
+                }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    f32x16 t;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) t[r] = 0.f;
+#pragma unroll
+                    for (int q = 0; q < kTerms; ++q)
+                        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kTermA[q]][i], d[kTermB[q]][j], t, 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], d[0][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] += t;
+                }
         }
     }
-    float *p = part + (size_t)blockIdx.x * H * H;
+    if (__syncthreads_or(top >= kSplitTop)) {  // a value that does not split: FP32 sums
+        const float *S = op ? B : A;
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) p[(size_t)(wave * 32 + acc_row(r, lane)) * H + b * 32 + (lane & 31)] = acc[b][r];
-}
-
-// Small products on the vector ALUs: partial of G[K, C] = A[rows, K]^T D[rows, C]
-// for K, C <= 128 (input layer, output layer, bias rows with A = 1).
-__global__ void __launch_bounds__(kThreads) k_small_grad_part(const float *__restrict__ A, int K,
-                                                              const float *__restrict__ D, int C, int N,
-                                                              float *__restrict__ part)
-{
-    const int r0 = blockIdx.x * kRowChunk;
-    const int r1 = (r0 + kRowChunk < N) ? r0 + kRowChunk : N;
-    float *p = part + (size_t)blockIdx.x * K * C;
-    for (int e = threadIdx.x; e < K * C; e += kThreads) {
-        const int k = e / C, c = e % C;
-        float s = 0.f;
-#pragma unroll 8
-        for (int r = r0; r < r1; ++r) s += (A ? A[(size_t)r * K + k] : 1.f) * D[(size_t)r * C + c];
-        p[e] = s;
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int row = wr + 32 * i + acc_row(r, lane), col = wc + 32 * j + (lane & 31);
+                    float v = 0.f;
+                    for (int n = r0; n < r1; ++n) v = fmaf(S[(size_t)n * H + row], D[(size_t)n * H + col], v);
+                    acc[i][j][r] = v;
+                }
     }
+    float *p = part + (size_t)blockIdx.x * kGradOut;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                p[op * H * H + (wr + 32 * i + acc_row(r, lane)) * H + wc + 32 * j + (lane & 31)] = acc[i][j][r];
+    float *red = reinterpret_cast<float *>(T);  // [4][H]; every read of T is behind the barrier above
+    red[g * H + f] = colSum;
+    __syncthreads();
+    if (g == 0) p[2 * H * H + f] = (red[f] + red[H + f]) + (red[2 * H + f] + red[3 * H + f]);
 }
 
-// out = sum of nPart partials of size n.  A workgroup owns 64 consecutive
-// outputs (lane = output); wave w adds partials w, w + 4, w + 8, .. in order
-// and the four wave sums are added in wave order: a fixed order, so the
-// result is deterministic.
-constexpr int kSumWaves = kThreads / 64;
-__global__ void __launch_bounds__(kThreads) k_sum_parts(const float *__restrict__ part, int nPart, int n,
-                                                        float *__restrict__ out)
+// The gradients of the input and the output layer: partials over `rows` rows
+// of V^T M [KS, 128] for M [N, 128] and V [N, KS], thread = a column of M and
+// every other row (a row of V is the same for a whole wave).
+// Input layer (SUMS 0): G[k][c] as it is, then the column sums of M.
+// Output layer (SUMS 1): G as [c][k], then the column sums of V.
+template <int KS, int SUMS>
+__global__ void __launch_bounds__(kThreads) k_edge_grad_part(const float *__restrict__ M, const float *__restrict__ V,
+                                                             int N, int rows, float *__restrict__ part)
 {
-    __shared__ float red[kSumWaves][64];
+    constexpr int nOut = KS * H + (SUMS ? KS : H);
+    __shared__ float red[nOut];
+    const int c = threadIdx.x & (H - 1), half = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 7);
+    const int r0 = blockIdx.x * rows, r1 = min(r0 + rows, N);
+    float s[KS], sv[KS], sm = 0.f;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) s[k] = sv[k] = 0.f;
+#pragma unroll 8
+    for (int r = r0 + half; r < r1; r += 2) {
+        const float x = M[(size_t)r * H + c];
+        sm += x;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            const float v = V[(size_t)r * KS + k];
+            s[k] = fmaf(v, x, s[k]);
+            if (SUMS) sv[k] += v;
+        }
+    }
+    if (half) {
+#pragma unroll
+        for (int k = 0; k < KS; ++k) red[SUMS ? c * KS + k : k * H + c] = s[k];
+        if (!SUMS) red[KS * H + c] = sm;
+        else if (c == 0)
+#pragma unroll
+            for (int k = 0; k < KS; ++k) red[KS * H + k] = sv[k];
+    }
+    __syncthreads();
+    if (half) return;
+    float *p = part + (size_t)blockIdx.x * nOut;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const int e = SUMS ? c * KS + k : k * H + c;
+        p[e] = s[k] + red[e];
+    }
+    if (!SUMS) p[KS * H + c] = sm + red[KS * H + c];
+    else if (c == 0)
+#pragma unroll
+        for (int k = 0; k < KS; ++k) p[KS * H + k] = sv[k] + red[KS * H + k];
+}
+inline __host__ __device__ int edge_rows(int N)
+{
+    const int r = (N + 1023) / 1024;
+    return r < 64 ? 64 : (r < kRowChunk ? r : kRowChunk);
+}
+
+// Sums of nPart partials of n values, written in up to three runs (the first
+// n0 values to o0, the next n1 to o1, the rest to o2).  A workgroup owns 64
+// consecutive values (lane = value); wave w adds partials w, w + 4, w + 8, ..
+// in order and the four wave sums are added in wave order: a fixed order, so
+// the result is deterministic.  The partials are many and their sum long, so
+// it is kept in FP64 (free: the kernel is bound by reading them).
+constexpr int kSumWaves = kThreads / 64;
+__global__ void __launch_bounds__(kThreads) k_sum_parts(const float *__restrict__ part, int nPart, int n, int n0,
+                                                        int n1, float *__restrict__ o0, float *__restrict__ o1,
+                                                        float *__restrict__ o2)
+{
+    __shared__ double red[kSumWaves][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int e = blockIdx.x * 64 + lane;
-    float s = 0.f;
+    double s = 0.0;
     if (e < n)
-        for (int i = wave; i < nPart; i += kSumWaves) s += part[(size_t)i * n + e];
+#pragma unroll 8
+        for (int i = wave; i < nPart; i += kSumWaves) s += double(part[(size_t)i * n + e]);
     red[wave][lane] = s;
     __syncthreads();
     if (wave == 0 && e < n) {
-        float t = red[0][lane];
-        for (int w = 1; w < kSumWaves; ++w) t += red[w][lane];
-        out[e] = t;
+        double d = red[0][lane];
+        for (int w = 1; w < kSumWaves; ++w) d += red[w][lane];
+        const float t = float(d);
+        if (e < n0) o0[e] = t;
+        else if (e < n0 + n1) o1[e - n0] = t;
+        else o2[e - n0 - n1] = t;
     }
 }
 
@@ -627,20 +747,34 @@ void dense(const Product &p1, const Product &p2, bool transpose, const float *bi
     else hipLaunchKernelGGL(k_dense<1>, g, b, 0, s, p1, p2, transpose, bias, N, mode, Hres, Z, out);
 }
 
-int grad_parts(int N) { return nb(N, kRowChunk); }
-
-void wgrad(const float *A, const float *D, int N, float *part, float *out, hipStream_t s)
+size_t grad_floats(int N)
 {
-    const int np = grad_parts(N);
-    hipLaunchKernelGGL(k_wgrad_part, dim3(np), dim3(kThreads), 0, s, A, D, N, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(nb(H * H, 64)), dim3(kThreads), 0, s, part, np, H * H, out);
+    const size_t w = (size_t)nb(N, grad_rows(N)) * kGradOut, e = (size_t)nb(N, edge_rows(N)) * ((kIn + 1) * H);
+    static_assert(kOut * H + kOut <= (kIn + 1) * H, "the input layer's partials are the larger");
+    return w > e ? w : e;
 }
 
-void small_grad(const float *A, int K, const float *D, int C, int N, float *part, float *out, hipStream_t s)
+void wgrad(const float *A, const float *B, const float *D, int N, float *part, float *gA, float *gB, float *gc,
+           hipStream_t s)
 {
-    const int np = grad_parts(N);
-    hipLaunchKernelGGL(k_small_grad_part, dim3(np), dim3(kThreads), 0, s, A, K, D, C, N, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(nb(K * C, 64)), dim3(kThreads), 0, s, part, np, K * C, out);
+    const int rows = grad_rows(N), np = nb(N, rows);
+    hipLaunchKernelGGL(k_wgrad_part, dim3(np), dim3(kGradThreads), 0, s, A, B, D, N, rows, part);
+    hipLaunchKernelGGL(k_sum_parts, dim3(nb(kGradOut, 64)), dim3(kThreads), 0, s, part, np, kGradOut, H * H, H * H, gA,
+                       gB, gc);
+}
+
+void input_grad(const float *X, const float *D, int N, float *part, float *gW0, float *gb0, hipStream_t s)
+{
+    const int rows = edge_rows(N), np = nb(N, rows), n = (kIn + 1) * H;
+    hipLaunchKernelGGL((k_edge_grad_part<kIn, 0>), dim3(np), dim3(kThreads), 0, s, D, X, N, rows, part);
+    hipLaunchKernelGGL(k_sum_parts, dim3(nb(n, 64)), dim3(kThreads), 0, s, part, np, n, kIn * H, H, gW0, gb0, gb0);
+}
+
+void output_grad(const float *h, const float *dy, int N, float *part, float *gWo, float *gbo, hipStream_t s)
+{
+    const int rows = edge_rows(N), np = nb(N, rows), n = kOut * H + kOut;
+    hipLaunchKernelGGL((k_edge_grad_part<kOut, 1>), dim3(np), dim3(kThreads), 0, s, h, dy, N, rows, part);
+    hipLaunchKernelGGL(k_sum_parts, dim3(nb(n, 64)), dim3(kThreads), 0, s, part, np, n, kOut * H, kOut, gWo, gbo, gbo);
 }
 
 void neighbour_mean(const int *nbr, int W, int N, const float *invDeg, const float *h, float *m, hipStream_t s)

@@ -95,7 +95,7 @@ phl_status alloc_activations(phl_mpnn *n)
     TRY(dev_alloc(n->act, &n->dh2, NH));
     TRY(dev_alloc(n->act, &n->dz, NH));
     TRY(dev_alloc(n->act, &n->dm, NH));
-    TRY(dev_alloc(n->act, &n->part, (size_t)phl::nn::grad_parts(n->N) * kHidden * kHidden));
+    TRY(dev_alloc(n->act, &n->part, phl::nn::grad_floats(n->N)));
     TRY(dev_alloc(n->act, &n->lossPart, (size_t)phl::nn::loss_parts(n->N * kOut)));
     TRY(dev_alloc(n->act, &n->lossOut, 1));
     return PHL_OK;
@@ -139,15 +139,13 @@ void backward(phl_mpnn *n)
     hipStream_t s = n->stream;
     const int N = n->N;
     const size_t NH = (size_t)N * kHidden, HH = (size_t)kHidden * kHidden;
-    small_grad(n->hs + NH * n->L, kHidden, n->dy, kOut, N, n->part, n->g + n->oWo, s);
-    small_grad(nullptr, 1, n->dy, kOut, N, n->part, n->g + n->obo, s);
+    output_grad(n->hs + NH * n->L, n->dy, N, n->part, n->g + n->oWo, n->g + n->obo, s);
     out_layer_back(n->dy, n->p + n->oWo, N, n->dh, s);
     split_weights(n->p + n->oA, n->p + n->oB, n->L, 3, true, n->wt16, n->wtBad, s);
     for (int l = n->L - 1; l >= 0; --l) {
         relu_back(n->dh, n->zs + NH * l, NH, n->dz, s);
-        wgrad(n->hs + NH * l, n->dz, N, n->part, n->g + n->oA + HH * l, s);
-        wgrad(n->ms + NH * l, n->dz, N, n->part, n->g + n->oB + HH * l, s);
-        small_grad(nullptr, 1, n->dz, kHidden, N, n->part, n->g + n->oc + kHidden * l, s);
+        wgrad(n->hs + NH * l, n->ms + NH * l, n->dz, N, n->part, n->g + n->oA + HH * l, n->g + n->oB + HH * l,
+              n->g + n->oc + kHidden * l, s);
         // dm = dz B^T;  dh' = dh + dz A^T + (mean)^T dm
         const Product none{};
         dense(hidden_product(n, n->dz, l, 1, 3), none, true, nullptr, N, 0, nullptr, nullptr, n->dm, 3, s);
@@ -156,8 +154,7 @@ void backward(phl_mpnn *n)
         std::swap(n->dh, n->dh2);
     }
     relu_back(n->dh, n->z0, NH, n->dz, s);
-    small_grad(n->X, kIn, n->dz, kHidden, N, n->part, n->g + n->oW0, s);
-    small_grad(nullptr, 1, n->dz, kHidden, N, n->part, n->g + n->ob0, s);
+    input_grad(n->X, n->dz, N, n->part, n->g + n->oW0, n->g + n->ob0, s);
 }
 
 }  // namespace

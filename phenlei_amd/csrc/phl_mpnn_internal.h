@@ -32,11 +32,15 @@ struct Product {
 // the kernel): FP32 products (3 pieces) or BF16 ones (1), FP32 accumulation.
 void dense(const Product &p1, const Product &p2, bool transpose, const float *bias, int N, int mode,
            const float *Hres, float *Z, float *out, int pieces, hipStream_t s);
-int grad_parts(int N);
-// out[128,128] = A[N,128]^T D[N,128] (part: grad_parts(N) * 128 * 128 floats)
-void wgrad(const float *A, const float *D, int N, float *part, float *out, hipStream_t s);
-// out[K,C] = A[N,K]^T D[N,C] (A null: a column of ones, K = 1)
-void small_grad(const float *A, int K, const float *D, int C, int N, float *part, float *out, hipStream_t s);
+// Weight gradients; part: grad_floats(N) floats of workspace.
+size_t grad_floats(int N);
+// gA = A^T D, gB = B^T D [128,128] and gc = the column sums of D, all [N,128].
+void wgrad(const float *A, const float *B, const float *D, int N, float *part, float *gA, float *gB, float *gc,
+           hipStream_t s);
+// gW0[8,128] = X^T D, gb0 = the column sums of D.
+void input_grad(const float *X, const float *D, int N, float *part, float *gW0, float *gb0, hipStream_t s);
+// gWo[128,5] = h^T dy, gbo = the column sums of dy.
+void output_grad(const float *h, const float *dy, int N, float *part, float *gWo, float *gbo, hipStream_t s);
 void neighbour_mean(const int *nbr, int W, int N, const float *invDeg, const float *h, float *m, hipStream_t s);
 void neighbour_mean_transpose_add(const int *nbr, int W, int N, const float *invDeg, const float *dm, float *dh,
                                   hipStream_t s);
