@@ -204,16 +204,18 @@ void build_sweep_order(int nC, const std::vector<int> &c2fPtr, const std::vector
 }
 
 // The dataflow sweep's order (phl::FlowOrder) for one direction: each level
-// of `cells` (mesh numbers, level order) padded to whole chunks of 64
-// positions, and the slot lists of build_sweep_order moved along (row, nb in
+// of `cells` (mesh numbers, level order) padded to whole chunks (64 positions,
+// or 16 in the quad form), and the slot lists of build_sweep_order moved along (row, nb in
 // mesh numbers; converted to storage here), the boundary faces, which come
 // first in every list, apart from the real neighbours.
 phl_status build_flow_order(phl_ctx *c, int nC, const std::vector<int> &cells, const std::vector<int> &lptr,
                             const std::vector<int> &row, const std::vector<int> &nb, int Wa,
                             const std::vector<int> &slotOf, phl::FlowOrder &fo)
 {
+    const bool quad = nC <= (long long)phl::kQuadLevel * ((long long)lptr.size() - 1);
+    const int CS = quad ? 16 : 64;  // cells per chunk
     int nCh = 0, W = 0, WG = 0;
-    for (size_t L = 0; L + 1 < lptr.size(); ++L) nCh += (lptr[L + 1] - lptr[L] + 63) / 64;
+    for (size_t L = 0; L + 1 < lptr.size(); ++L) nCh += (lptr[L + 1] - lptr[L] + CS - 1) / CS;
     for (int pos = 0; pos < nC; ++pos) {
         int g = 0, n = 0;
         for (int s = 0; s < Wa && row[(size_t)s * nC + pos] >= 0; ++s) ++(nb[(size_t)s * nC + pos] >= nC ? g : n);
@@ -221,16 +223,17 @@ phl_status build_flow_order(phl_ctx *c, int nC, const std::vector<int> &cells, c
         WG = std::max(WG, g);
     }
     W = W <= 3 ? 3 : (W <= 4 ? 4 : 6);
-    const size_t Pp = (size_t)64 * nCh;
-    std::vector<int> fc(Pp, -1), frow((size_t)W * Pp, -1), fnb((size_t)W * Pp, 0), frowG((size_t)WG * Pp, -1);
+    const size_t Pp = (size_t)CS * nCh, slots = quad ? (W <= 4 ? 4 : 8) : W;
+    std::vector<int> fc(Pp, -1), frow(slots * Pp, -1), fnb(slots * Pp, 0), frowG((size_t)WG * Pp, -1);
+    auto at = [&](int s, size_t q) { return quad ? ((s / 4) * Pp + q) * 4 + s % 4 : s * Pp + q; };
     std::vector<int> chunkOf(nC, -1), width(std::max(nCh, 1), 0), widthG(std::max(nCh, 1), 0);
     int ch = 0;
     for (size_t L = 0; L + 1 < lptr.size(); ++L) {
         const int levelChunk0 = ch;
-        for (int b = lptr[L]; b < lptr[L + 1]; b += 64, ++ch) {
-            for (int j = 0; j < 64 && b + j < lptr[L + 1]; ++j) {
+        for (int b = lptr[L]; b < lptr[L + 1]; b += CS, ++ch) {
+            for (int j = 0; j < CS && b + j < lptr[L + 1]; ++j) {
                 const int pos = b + j;
-                const size_t q = (size_t)ch * 64 + j;
+                const size_t q = (size_t)ch * CS + j;
                 fc[q] = slotOf[cells[pos]];
                 chunkOf[cells[pos]] = ch;
                 int g = 0, n = 0;
@@ -245,8 +248,8 @@ phl_status build_flow_order(phl_ctx *c, int nC, const std::vector<int> &cells, c
                     // a neighbour swept earlier lies in a chunk of an earlier level
                     if (chunkOf[o] < 0 || chunkOf[o] >= levelChunk0)
                         return fail(PHL_ERR_ARG, "dataflow sweep order: a neighbour is not in an earlier level");
-                    frow[(size_t)n * Pp + q] = r;
-                    fnb[(size_t)n++ * Pp + q] = slotOf[o];
+                    frow[at(n, q)] = r;
+                    fnb[at(n++, q)] = slotOf[o];
                 }
                 width[ch] = std::max(width[ch], n);
                 widthG[ch] = std::max(widthG[ch], g);
@@ -260,7 +263,7 @@ phl_status build_flow_order(phl_ctx *c, int nC, const std::vector<int> &cells, c
     {
         int ch0 = 0;
         for (size_t L = 0; L + 1 < lptr.size(); ++L) {
-            const int nL = (lptr[L + 1] - lptr[L] + 63) / 64, g = (nL + 7) / 8;
+            const int nL = (lptr[L + 1] - lptr[L] + CS - 1) / CS, g = (nL + 7) / 8;
             for (int j = 0; j < g; ++j)
                 for (int x = 0; x < 8; ++x) blockChunk.push_back(x * g + j < nL ? ch0 + x * g + j : -1);
             ch0 += nL;
@@ -280,6 +283,7 @@ phl_status build_flow_order(phl_ctx *c, int nC, const std::vector<int> &cells, c
     TRY(upload(c, &t, blockChunk)); fo.blockChunk = t;
     fo.nBlocks = (int)blockChunk.size();
     fo.W = W;
+    fo.quad = quad;
     fo.nChunks = nCh;
     return PHL_OK;
 }

@@ -222,16 +222,28 @@ struct SweepOrder {
 };
 
 // Dataflow sweep order: the level order with every level padded to whole
-// chunks of 64 positions (a chunk never spans two levels), so a chunk
-// depends only on chunks of earlier levels.
+// chunks (a chunk never spans two levels), so a chunk depends only on chunks
+// of earlier levels.  A chunk is a wavefront's: 64 cells, one per lane, or
+// (quad) 16 cells of four lanes each.
+// The quad form shortens the chain (a level's arithmetic is one slot's, not
+// three to six in a row) for about a third more instructions, so it is taken
+// while levels are narrow.  Sweeps per step (forward + backward), 64 cells per
+// wavefront against 16: hex channel of 512 cells (20 per level) 0.050 + 0.055
+// ms against 0.036 + 0.040, 16k (160) 0.195 + 0.200 against 0.141 + 0.147,
+// 254k (1,100) 0.50 + 0.50 against 0.35 + 0.34, wing of 2.24M (6,200) 0.90 +
+// 1.04 against 0.81 + 0.83; batches with 10,300 per level 0.92 + 0.93 against
+// 0.74 + 0.82, with 19,300 1.20 + 1.24 against 1.14 + 1.31, with 29,300 1.53 +
+// 1.63 against 1.62 + 1.89.
+constexpr int kQuadLevel = 18000;  // cells per level up to which the quad form is built
 struct FlowOrder {
     int nChunks;        // 0: not built
-    int W;              // slots per position: 3, 4 or 6
-    const int *cells;   // [64*nChunks] storage index, -1 for padding
-    const int *row;     // [W][64*nChunks] as SweepOrder::row, real neighbours only
-    const int *nb;      // [W][64*nChunks] as SweepOrder::nb
+    bool quad;
+    int W;              // slots per position: 3, 4 or 6 (quad: lists hold 4 or 8)
+    const int *cells;   // [positions] storage index, -1 for padding
+    const int *row;     // [W][positions] as SweepOrder::row, real neighbours only (quad: [W/4][positions][4])
+    const int *nb;      // as row: SweepOrder::nb
     const int *width;   // [nChunks] most active slots of any cell of the chunk (slots are packed first)
-    const int *rowG;    // [most][64*nChunks] rows of the boundary faces (backward sweep; -1 pad), or null
+    const int *rowG;    // [most][positions] rows of the boundary faces (backward sweep; -1 pad), or null
     const int *widthG;  // [nChunks] most boundary faces of any cell of the chunk
     // sweep_form 3: block i sweeps chunk blockChunk[i] (-1: nothing).  Each
     // level's chunks are split into 8 contiguous groups, group x going to the

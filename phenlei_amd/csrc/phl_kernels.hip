@@ -2085,8 +2085,9 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_block_so(DevMesh M, Const
 
 // ------------------------------------------------- dataflow sweep
 // One launch per direction instead of one per level (sweep_form 0, 2 and 3).
-// A wavefront sweeps one chunk of 64 positions of the padded level order; a
-// chunk depends only on chunks of earlier levels, which earlier blocks hold.
+// A wavefront sweeps one chunk of the padded level order (64 positions, or 16
+// in the quad form, see FlowOrder); a chunk depends only on chunks of earlier
+// levels, which earlier blocks hold.
 //
 // The increments themselves say when they are there.  Every sweep writes the
 // one of two dq buffers that holds kMark in every real row, and marks the
@@ -2103,7 +2104,7 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_block_so(DevMesh M, Const
 // took 1.53 + 1.56 ms on the 2.24M-cell wing, 0.99 + 0.99 on the 1.01M-cell
 // hybrid channel, 0.60 + 0.63 on the 254k-cell and 0.23 + 0.27 on the 16k-cell
 // hex channel; marks take 0.90 + 1.04, 0.55 + 0.57, 0.50 + 0.50 and 0.20 +
-// 0.20.  A flag published early as a hint, before polling the rows, was slower
+// 0.20 (64 cells per wavefront).  A flag published early as a hint, before polling the rows, was slower
 // than polling at once (wing 1.10 + 1.22).
 // Polling the rows pays only because they are few lines: storage follows the
 // level order (sweep_order), so the 64 neighbours of a slot lie in short runs
@@ -2325,6 +2326,169 @@ __device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, co
     return true;
 }
 
+// The same with four lanes per cell (16 cells per wavefront): lane j of a
+// quad takes slots j, j + 4, .. of its cell, the quad adds the terms in slot
+// order (DPP broadcasts), and lane j makes the j-th value of the row (lane 0
+// also the fifth, lane 1 the Spalart-Allmaras increment).  Same operations
+// and order, so the same bits.
+__device__ __forceinline__ double quad_get(double v, int j)
+{
+    const long long b = __double_as_longlong(v);
+    int lo = (int)b, hi = (int)(b >> 32);
+    switch (j) {
+    case 0: lo = __builtin_amdgcn_mov_dpp(lo, 0x00, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0x00, 0xf, 0xf, true); break;
+    case 1: lo = __builtin_amdgcn_mov_dpp(lo, 0x55, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0x55, 0xf, 0xf, true); break;
+    case 2: lo = __builtin_amdgcn_mov_dpp(lo, 0xaa, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0xaa, 0xf, 0xf, true); break;
+    default: lo = __builtin_amdgcn_mov_dpp(lo, 0xff, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0xff, 0xf, 0xf, true); break;
+    }
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <int NG, int VIS, typename CT>
+__device__ __forceinline__ bool flow_quad(const DevMesh &M, const Consts &K, const FlowOrder &fo, const int *ctl,
+                                          bool useU, const double *__restrict__ coef, const double *__restrict__ res,
+                                          const double *__restrict__ diag, double *dq, double *dqOld, double *dflux,
+                                          const SaSweep &sa, const GatherRec *__restrict__ rec,
+                                          const double *__restrict__ vist, int tk, int lane, long long t0,
+                                          long long waitTicks)
+{
+    const int nT = M.nTotal, nC = M.nCell, P = 16 * fo.nChunks;
+    const int p = tk * 16 + (lane >> 2), j = lane & 3;
+    const int c = fo.cells[p];
+    const bool live = c >= 0, saLane = sa.on && j == 1;
+    const int cc = live ? c : 0;
+    const int width = __builtin_amdgcn_readfirstlane(fo.width[tk]);
+    int row[NG], nb[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        row[g] = -1;
+        nb[g] = 0;
+        if (4 * g < width) {
+            row[g] = fo.row[((size_t)g * P + p) * 4 + j];
+            nb[g] = fo.nb[((size_t)g * P + p) * 4 + j];
+        }
+    }
+    // the lane's two values: component j, and the fifth (lane 0) or SA (lane 1)
+    const double r1 = res[(size_t)j * nC + cc], r2 = saLane ? sa.res[cc] : res[(size_t)4 * nC + cc];
+    const double D1 = diag[cc], D2 = saLane ? sa.spec[cc] : D1;
+    double U1 = 0.0, U2 = 0.0;
+    if (useU) {
+        U1 = reinterpret_cast<const double *>(pair_at(dflux, nC, cc, j >> 1))[j & 1];
+        U2 = pair_at(dflux, nC, cc, 2)->x;
+    }
+    if (saLane) U2 = sa.dflux[cc];
+    double co[NG][16];
+    Consts Kc = K;
+    double qc[5], xc[3], vc = 0.0;
+    if (K.coefInSweep) {
+        Kc = case_k(K, M, cc);
+        load_rec_state(rec, cc, qc, xc);
+        vc = vist[cc];
+    }
+    double aT[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        aT[g] = 0.0;
+        if (4 * g >= width) break;
+        const int rw = row[g] >= 0 ? row[g] : 0;
+        if (K.coefInSweep) side_coef<CT>(M, Kc, rec, vist, qc, xc, vc, rw, row[g] >= 0 ? nb[g] : cc, co[g]);
+        else load_coef_row<CT>(coef, rw, co[g]);
+        if (sa.on) aT[g] = sa.mat[rw];
+    }
+    const __amdgpu_buffer_rsrc_t dqr = __builtin_amdgcn_make_buffer_rsrc(
+        dq, 0, (int)((size_t)nT * kPlanes * sizeof(double2)), kRawBufferWord3);
+    const int plane = nT * (int)sizeof(double2);
+    // terms of ghost neighbours (see flow_chunk), in lane 0
+    double rhs[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const int widthG = fo.rowG ? __builtin_amdgcn_readfirstlane(fo.widthG[tk]) : 0;
+    for (int s = 0; s < widthG; ++s) {
+        const int rw = j == 0 ? fo.rowG[(size_t)s * P + p] : -1;
+        if (rw < 0) continue;
+        const int gh = nC + (rw >> 1);
+        double cg[16], dg[5], df[5];
+        if (K.coefInSweep) side_coef<CT>(M, Kc, rec, vist, qc, xc, vc, rw, gh, cg);
+        else load_coef_row<CT>(coef, rw, cg);
+        load_row5(dq, nT, gh, dg);
+        sweep_apply<VIS>(K, cg, dg, df);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) rhs[m] += df[m];
+        if (sa.on) rhs[5] += sa.mat[rw] * pair_at(dq, nT, gh, 2)->y;
+    }
+    if (widthG > 0) {
+#pragma unroll
+        for (int m = 0; m < 6; ++m) rhs[m] = quad_get(rhs[m], 0);
+    }
+
+    v4i x[NG], y[NG], z[NG];
+    bool wait[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        wait[g] = row[g] >= 0;
+        x[g] = y[g] = z[g] = v4i{0, 0, 0, 0};
+    }
+    for (int it = 1;; ++it) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            if (4 * g >= width) break;
+            if (wait[g]) {
+                const int o = nb[g] * (int)sizeof(double2);
+                x[g] = __builtin_amdgcn_raw_buffer_load_b128(dqr, o, 0, kDeviceScope);
+                y[g] = __builtin_amdgcn_raw_buffer_load_b128(dqr, o + plane, 0, kDeviceScope);
+                z[g] = __builtin_amdgcn_raw_buffer_load_b128(dqr, o + 2 * plane, 0, kDeviceScope);
+            }
+        }
+        bool again = false;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            if (4 * g >= width) break;
+            wait[g] = wait[g] && (((x[g][0] & x[g][1]) == -1) | ((x[g][2] & x[g][3]) == -1) |
+                                  ((y[g][0] & y[g][1]) == -1) | ((y[g][2] & y[g][3]) == -1) |
+                                  ((z[g][0] & z[g][1]) == -1) | (sa.on & ((z[g][2] & z[g][3]) == -1)));
+            again = again || wait[g];
+        }
+        if (!__any(again)) break;
+        if (wall_clock64() - t0 > waitTicks || ((it & 63) == 0 && ctl_load(&ctl[2]) != 0)) return false;
+        __builtin_amdgcn_s_sleep(1);
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (4 * g >= width) break;
+        const double2 a = __builtin_bit_cast(double2, x[g]), b = __builtin_bit_cast(double2, y[g]),
+                      d = __builtin_bit_cast(double2, z[g]);
+        const double dqn[5] = {a.x, a.y, b.x, b.y, d.x};
+        double df[6];
+        sweep_apply<VIS>(K, co[g], dqn, df);
+        df[5] = aT[g] * d.y;
+        const bool act = row[g] >= 0;
+#pragma unroll
+        for (int m = 0; m < 6; ++m) df[m] = act ? df[m] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (4 * g + q >= width) break;
+#pragma unroll
+            for (int m = 0; m < 5; ++m) rhs[m] += quad_get(df[m], q);
+            if (sa.on) rhs[5] += quad_get(df[5], q);
+        }
+    }
+    if (live) {
+        const double s1 = j == 0 ? rhs[0] : (j == 1 ? rhs[1] : (j == 2 ? rhs[2] : rhs[3])), s2 = saLane ? rhs[5] : rhs[4];
+        const double v1 = not_mark((r1 - U1 - s1) / D1), v2 = not_mark((r2 - U2 - s2) / D2);
+        const int o = c * (int)sizeof(double2) + 8 * (j & 1);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, v1), dqr, o + (j >> 1) * plane, 0, kDeviceScope);
+        if (j == 0 || saLane)
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, v2), dqr, o + 2 * plane, 0, kDeviceScope);
+        reinterpret_cast<double *>(pair_at(dflux, nC, c, j >> 1))[j & 1] = 0.0 + s1;
+        if (j == 0) pair_at(dflux, nC, c, 2)->x = 0.0 + s2;
+        if (saLane) {
+            sa.dflux[c] = 0.0 + s2;
+            sa.dq[c] = v2;
+        }
+        const double mark = __longlong_as_double((long long)kMark);
+        if (j < kPlanes) *pair_at(dqOld, nT, c, j) = make_double2(mark, mark);
+    }
+    return true;
+}
+
 // TICKET false (sweep_form 0): block b sweeps chunk b; (sweep_form 3) block b
 // sweeps chunk blockChunk[b], the levels' chunks split into eighths over the
 // XCDs (block ids still rise with the level).  Workgroups of a
@@ -2335,7 +2499,7 @@ __device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, co
 // chunks from a ticket counter, so a chunk is only ever claimed by a running
 // block after every smaller chunk, whatever the dispatch order (the counter
 // is one device-scope atomic per block, which serialises large launches).
-template <int NW, int VIS, typename CT, bool TICKET>
+template <int NW, bool QUAD, int VIS, typename CT, bool TICKET>
 __global__ void __launch_bounds__(TICKET ? 256 : 64) k_sweep_flow(DevMesh M, Consts K, FlowOrder fo, int *ctl,
                                                                   bool useU, const double *__restrict__ coef,
                                                                   const double *__restrict__ res, const double *__restrict__ diag, double *dq,
@@ -2357,9 +2521,14 @@ __global__ void __launch_bounds__(TICKET ? 256 : 64) k_sweep_flow(DevMesh M, Con
     } else {
         tk = blockIdx.x;
     }
-    if (!flow_chunk<NW, VIS, CT>(M, K, fo, ctl, useU, coef, res, diag, dq, dqOld, dflux, sa, rec, vist, tk, lane,
-                                 wall_clock64(), (long long)ctl[3]))
-        if (lane == 0) atomicAdd(&ctl[2], 1);
+    bool done;
+    if constexpr (QUAD)
+        done = flow_quad<NW, VIS, CT>(M, K, fo, ctl, useU, coef, res, diag, dq, dqOld, dflux, sa, rec, vist, tk, lane,
+                                      wall_clock64(), (long long)ctl[3]);
+    else
+        done = flow_chunk<NW, VIS, CT>(M, K, fo, ctl, useU, coef, res, diag, dq, dqOld, dflux, sa, rec, vist, tk, lane,
+                                       wall_clock64(), (long long)ctl[3]);
+    if (!done && lane == 0) atomicAdd(&ctl[2], 1);
 }
 
 // Ghost dq from the forward sweep's dq, into the buffer the backward sweep
@@ -2915,7 +3084,7 @@ void launch_mark_dq(const DevMesh &m, double *dq, hipStream_t s)
                        reinterpret_cast<unsigned long long *>(dq), n);
 }
 
-template <int NW, int VIS, typename CT>
+template <int NW, bool QUAD, int VIS, typename CT>
 static void launch_sweep_flow(const DevMesh &m, const Consts &k, DevFlow &f, const FlowOrder &fo, bool useU,
                               bool withSA, hipStream_t s)
 {
@@ -2924,25 +3093,25 @@ static void launch_sweep_flow(const DevMesh &m, const Consts &k, DevFlow &f, con
     std::swap(f.dq, f.dqAlt);  // the marked buffer becomes the current one
     if (k.sweepForm == 2) {
         hipLaunchKernelGGL(k_sweep_ticket, dim3(1), dim3(1), 0, s, f.sweepCtl);
-        hipLaunchKernelGGL((k_sweep_flow<NW, VIS, CT, true>), dim3(nblk(fo.nChunks, 4)), dim3(256), 0, s, m, k, fo,
+        hipLaunchKernelGGL((k_sweep_flow<NW, QUAD, VIS, CT, true>), dim3(nblk(fo.nChunks, 4)), dim3(256), 0, s, m, k, fo,
                            f.sweepCtl, useU, f.coef, f.res, f.diag, f.dq, f.dqAlt, f.dflux, sa, f.rec, f.vist);
     } else {
-        hipLaunchKernelGGL((k_sweep_flow<NW, VIS, CT, false>), dim3(k.sweepForm == 3 ? fo.nBlocks : fo.nChunks),
+        hipLaunchKernelGGL((k_sweep_flow<NW, QUAD, VIS, CT, false>), dim3(k.sweepForm == 3 ? fo.nBlocks : fo.nChunks),
                            dim3(64), 0, s, m, k, fo, f.sweepCtl, useU, f.coef, f.res, f.diag, f.dq, f.dqAlt, f.dflux,
                            sa, f.rec, f.vist);
     }
 }
 
-template <int NW>
+template <int NW, bool QUAD>
 static void launch_sweep_flow_w(const DevMesh &m, const Consts &k, DevFlow &f, const FlowOrder &fo, bool useU,
                                 bool withSA, hipStream_t s)
 {
     if (k.coefF32) {  // only set when both directions have at most 6 slots
-        if (k.viscous) launch_sweep_flow<NW, 1, float>(m, k, f, fo, useU, withSA, s);
-        else launch_sweep_flow<NW, 0, float>(m, k, f, fo, useU, withSA, s);
+        if (k.viscous) launch_sweep_flow<NW, QUAD, 1, float>(m, k, f, fo, useU, withSA, s);
+        else launch_sweep_flow<NW, QUAD, 0, float>(m, k, f, fo, useU, withSA, s);
     } else {
-        if (k.viscous) launch_sweep_flow<NW, 1, double>(m, k, f, fo, useU, withSA, s);
-        else launch_sweep_flow<NW, 0, double>(m, k, f, fo, useU, withSA, s);
+        if (k.viscous) launch_sweep_flow<NW, QUAD, 1, double>(m, k, f, fo, useU, withSA, s);
+        else launch_sweep_flow<NW, QUAD, 0, double>(m, k, f, fo, useU, withSA, s);
     }
 }
 
@@ -2973,9 +3142,14 @@ void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &l
     const bool useU = !(forward && firstSweep);
     const bool v = k.viscous != 0;
     if (lv.flow.nChunks > 0) {  // built unless sweep_form is 1
-        if (lv.flow.W == 3) return launch_sweep_flow_w<3>(m, k, f, lv.flow, useU, withSA, s);
-        if (lv.flow.W == 4) return launch_sweep_flow_w<4>(m, k, f, lv.flow, useU, withSA, s);
-        return launch_sweep_flow_w<6>(m, k, f, lv.flow, useU, withSA, s);
+        const FlowOrder &fo = lv.flow;
+        if (fo.quad) {
+            if (fo.W <= 4) return launch_sweep_flow_w<1, true>(m, k, f, fo, useU, withSA, s);
+            return launch_sweep_flow_w<2, true>(m, k, f, fo, useU, withSA, s);
+        }
+        if (fo.W == 3) return launch_sweep_flow_w<3, false>(m, k, f, fo, useU, withSA, s);
+        if (fo.W == 4) return launch_sweep_flow_w<4, false>(m, k, f, fo, useU, withSA, s);
+        return launch_sweep_flow_w<6, false>(m, k, f, fo, useU, withSA, s);
     }
     if (k.coefF32) {
         if (lv.so.Wpad == 3) return v ? launch_sweep_so<3, 1, float>(m, k, f, lv, useU, s) : launch_sweep_so<3, 0, float>(m, k, f, lv, useU, s);

@@ -1,8 +1,9 @@
 """Storage in sweep-level order and the dataflow sweeps over it, at the shapes
 where an order or a chunk can go wrong: one cell, levels of exactly 64 and of
 65 cells, one-cell levels, a random numbering (many short levels), a colour
-numbering (two to four levels of half the mesh), a batch.  Every comparison is
-bitwise: the order only moves where a cell's data live."""
+numbering (two levels of half the mesh, six lower neighbours), a wide one past
+the quad form's limit of cells per level, a batch.  Every comparison is bitwise:
+the order only moves where a cell's data live."""
 import numpy as np
 import pytest
 
@@ -26,18 +27,19 @@ def shapes():
         "levels_of_65": lambda: pa.Mesh.bump_hex(65, 70, 1),
         "hybrid_shuffled": shuffled,
         "hex_coloured": lambda: pa.Mesh.bump_hex(9, 7, 5).renumbered("colour"),
+        "two_wide_levels": lambda: pa.Mesh.bump_hex(101, 60, 7).renumbered("colour"),
         "batch": lambda: pa.Mesh.concat([pa.Mesh.bump_hex(5, 4, 3, h) for h in (0.02, 0.05)]),
     }
 
 
 def run(mesh, steps, **over):
-    base = dict(mach=0.5, cfl_start=2.0, cfl_end=2.0, viscous=1, reynolds=5e4, **over)
+    base = dict(dict(mach=0.5, cfl_start=2.0, cfl_end=2.0, viscous=1, reynolds=5e4), **over)
     p = pa.default_params(**base)
     s = pa.Solver(mesh, [p] * mesh.n_cases if mesh.n_cases > 1 else p)
     s.init_freestream()
     s.set_state(perturbed_state(mesh.n_total, mesh.n_cell, FREE, 5, amp=0.01))
     s.iterate(1, steps)
-    return {k: s.get_field(k) for k in ("q", "res", "dq", "delta_flux")}
+    return {k: s.get_field(k) for k in ("q", "res", "dq", "delta_flux") + (("nut", "dq_t") if over.get("viscous") == 3 else ())}
 
 
 @pytest.mark.parametrize("name", sorted(shapes()))
@@ -53,6 +55,23 @@ def test_sweep_level_storage_equals_mesh_storage(name):
 def test_dataflow_sweep_at_chunk_edges_equals_level_form(name, form):
     mesh = shapes()[name]()
     a, b = run(mesh, 4, sweep_form=form), run(mesh, 4, sweep_form=1)
+    for k in a:
+        assert np.array_equal(a[k], b[k]), (name, k)
+
+
+@pytest.mark.parametrize("form", [0, 2])
+@pytest.mark.parametrize("name", ["levels_of_65", "hex_coloured", "two_wide_levels"])
+def test_carried_turbulence_sweep_at_chunk_edges(name, form):
+    mesh = shapes()[name]()
+    a, b = (run(mesh, 4, sweep_form=f, viscous=3, cfl_start=0.5, cfl_end=0.5) for f in (form, 1))
+    for k in a:
+        assert np.array_equal(a[k], b[k]), (name, k)
+
+
+@pytest.mark.parametrize("name", ["hex_coloured", "two_wide_levels"])
+def test_mixed_form_at_chunk_edges(name):
+    mesh = shapes()[name]()
+    a, b = run(mesh, 4, sweep_form=0, precision=1), run(mesh, 4, sweep_form=1, precision=1)
     for k in a:
         assert np.array_equal(a[k], b[k]), (name, k)
 
