@@ -553,8 +553,14 @@ __global__ void __launch_bounds__(kBlock) k_face_node_mean(DevMesh M, const doub
 
 // ------------------------------------------------ gradients + limiter
 // GT is the storage type of the gradients: double, or float for the mixed
-// form (computed in FP64, stored rounded to FP32).
-template <typename GT, int BS>
+// form (computed in FP64, stored rounded to FP32).  COEF: the LU-SGS face
+// coefficients are stored too (level form); GGCELL: gradient 0 only.  Bound by
+// memory latency: with every form in one kernel (172 registers, two waves per
+// SIMD) and a face's loads behind the previous face's sums it took 0.48 ms on
+// the 2.24M-cell wing, 0.21 on the 1.01M-cell hybrid and 0.34 on a 1.42M-cell
+// hex batch; as it is 0.42, 0.18 and 0.26.
+constexpr int kGradW = 6;
+template <typename GT, int BS, bool COEF, bool GGCELL>
 __global__ void __launch_bounds__(BS) k_grad_lim(DevMesh M, Consts K0, const double *__restrict__ q,
                                                      GT *__restrict__ grad, GT *__restrict__ gradT,
                                                      double *__restrict__ lim, double *__restrict__ coef,
@@ -564,7 +570,9 @@ __global__ void __launch_bounds__(BS) k_grad_lim(DevMesh M, Consts K0, const dou
     const int c = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int nC = M.nCell, nT = M.nTotal;
     if (c >= nC) return;
-    const Consts K = case_k(K0, M, c);
+    Consts K = case_k(K0, M, c);
+    if constexpr (GGCELL) K.gradient = 0;
+    K.coefInSweep = COEF ? 0 : 1;
     double qc[5];
     load5(q, nT, c, qc);
     double gx[5], gy[5], gz[5];
@@ -573,7 +581,51 @@ __global__ void __launch_bounds__(BS) k_grad_lim(DevMesh M, Consts K0, const dou
     double tgx = 0.0, tgy = 0.0, tgz = 0.0;
     const double tc = qc[4] / (K.R * qc[0]);
     double rmin = qc[0], rmax = qc[0], pmin = qc[4], pmax = qc[4];
-    for (int s = 0; s < M.ellW; ++s) {
+    // Cells of at most kGradW faces (ggcell): every list entry, then every face
+    // and neighbour in flight together, so that a cell waits for memory twice
+    // instead of twice per face; the same terms in the same order.
+    int encW[kGradW], nbW[kGradW];
+    const bool together = GGCELL && !COEF && M.ellW <= kGradW;
+    if (together) {
+#pragma unroll
+        for (int s = 0; s < kGradW; ++s) {
+            encW[s] = s < M.ellW ? M.c2fEnc[(size_t)s * nC + c] : 0;
+            nbW[s] = s < M.ellW ? M.c2n[(size_t)s * nC + c] : c;
+            if (encW[s] == 0) nbW[s] = c;
+        }
+        double4 fn[kGradW];
+        double qn[kGradW][5];
+#pragma unroll
+        for (int s = 0; s < kGradW; ++s) {
+            const int e = encW[s];
+            fn[s] = *reinterpret_cast<const double4 *>(&M.face[e == 0 ? 0 : (e > 0 ? e : -e) - 1]);
+            load5(q, nT, nbW[s], qn[s]);
+        }
+#pragma unroll
+        for (int s = 0; s < kGradW; ++s) {
+            const bool act = encW[s] != 0, isL = encW[s] > 0;
+            const double nx = fn[s].x * fn[s].w, ny = fn[s].y * fn[s].w, nz = fn[s].z * fn[s].w;
+            auto add = [&](double &sum, double t) { sum = act ? (isL ? sum + t : sum - t) : sum; };
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                const double qfc = 0.5 * (qc[m] + qn[s][m]);
+                add(gx[m], qfc * nx);
+                add(gy[m], qfc * ny);
+                add(gz[m], qfc * nz);
+            }
+            if (K.viscous) {
+                const double tfc = 0.5 * (tc + qn[s][4] / (K.R * qn[s][0]));
+                add(tgx, tfc * nx);
+                add(tgy, tfc * ny);
+                add(tgz, tfc * nz);
+            }
+            if (act && nbW[s] < nC) {
+                rmin = dMIN(rmin, qn[s][0]); rmax = dMAX(rmax, qn[s][0]);
+                pmin = dMIN(pmin, qn[s][4]); pmax = dMAX(pmax, qn[s][4]);
+            }
+        }
+    }
+    for (int s = 0; s < M.ellW && !together; ++s) {
         const int enc = M.c2fEnc[(size_t)s * nC + c];
         if (enc == 0) break;
         const bool isL = enc > 0;
@@ -704,18 +756,32 @@ __global__ void __launch_bounds__(BS) k_grad_lim(DevMesh M, Consts K0, const dou
         epsP *= vf;
         l = 1.0;
         const double xc = M.xcc[c], yc = M.ycc[c], zc = M.zcc[c];
-        for (int s = 0; s < M.ellW; ++s) {
-            const int enc = M.c2fEnc[(size_t)s * nC + c];
-            if (enc == 0) break;
-            const int f = (enc > 0 ? enc : -enc) - 1;
-            const FaceRec fr = M.face[f];
-            const double dx = fr.xc - xc, dy = fr.yc - yc, dz = fr.zc - zc;
+        auto limit = [&](double dx, double dy, double dz) {
             const double dqR = gx[0] * dx + gy[0] * dy + gz[0] * dz;
             if (dqR > kSMALL) l = dMIN(l, venfun(dmaxR, dqR, epsR));
             else if (dqR < -kSMALL) l = dMIN(l, venfun(dminR, dqR, epsR));
             const double dqP = gx[4] * dx + gy[4] * dy + gz[4] * dz;
             if (dqP > kSMALL) l = dMIN(l, venfun(dmaxP, dqP, epsP));
             else if (dqP < -kSMALL) l = dMIN(l, venfun(dminP, dqP, epsP));
+        };
+        if (together) {
+            double fx[kGradW], fy[kGradW], fz[kGradW];
+#pragma unroll
+            for (int s = 0; s < kGradW; ++s) {
+                const int e = encW[s];
+                const FaceRec &fr = M.face[e == 0 ? 0 : (e > 0 ? e : -e) - 1];
+                fx[s] = fr.xc; fy[s] = fr.yc; fz[s] = fr.zc;
+            }
+#pragma unroll
+            for (int s = 0; s < kGradW; ++s)
+                if (encW[s] != 0) limit(fx[s] - xc, fy[s] - yc, fz[s] - zc);
+        } else {
+            for (int s = 0; s < M.ellW; ++s) {
+                const int enc = M.c2fEnc[(size_t)s * nC + c];
+                if (enc == 0) break;
+                const FaceRec fr = M.face[(enc > 0 ? enc : -enc) - 1];
+                limit(fr.xc - xc, fr.yc - yc, fr.zc - zc);
+            }
         }
         if (M.limZero[c]) l = 0.0;
     }
@@ -2884,19 +2950,32 @@ void launch_gamma_t(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s
     hipLaunchKernelGGL(k_gamma_t, dim3(nblk(m.nTotal, kBlock)), dim3(kBlock), 0, s, m, k, f.q, f.t, f.visl);
 }
 
-template <int BS>
-static void launch_grad_lim_t(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s, bool fp32, bool soa)
+template <int BS, bool COEF, bool GGCELL>
+static void launch_grad_lim_k(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s, bool fp32, bool soa)
 {
     // the gather records hold the gradient type of the context's face loop
     GatherRec *rec = (fp32 == (k.mixed != 0)) ? f.rec : nullptr;
+    if (fp32)
+        hipLaunchKernelGGL((k_grad_lim<float, BS, COEF, GGCELL>), dim3(nblk(m.nCell, BS)), dim3(BS), 0, s, m, k, f.q,
+                           f.gradF, f.gradTF, f.lim, f.coef, f.vist, rec, soa, f.faceQ);
+    else
+        hipLaunchKernelGGL((k_grad_lim<double, BS, COEF, GGCELL>), dim3(nblk(m.nCell, BS)), dim3(BS), 0, s, m, k, f.q,
+                           f.grad, f.gradT, f.lim, f.coef, f.vist, rec, soa, f.faceQ);
+}
+
+template <int BS>
+static void launch_grad_lim_t(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s, bool fp32, bool soa)
+{
     if (k.gradient == 2)  // ggnode: face means of the node values in place
         hipLaunchKernelGGL(k_face_node_mean, dim3(nblk(m.nFace, kBlock)), dim3(kBlock), 0, s, m, f.nodeQ, f.faceQ);
-    if (fp32)
-        hipLaunchKernelGGL((k_grad_lim<float, BS>), dim3(nblk(m.nCell, BS)), dim3(BS), 0, s, m, k, f.q, f.gradF,
-                           f.gradTF, f.lim, f.coef, f.vist, rec, soa, f.faceQ);
-    else
-        hipLaunchKernelGGL((k_grad_lim<double, BS>), dim3(nblk(m.nCell, BS)), dim3(BS), 0, s, m, k, f.q, f.grad,
-                           f.gradT, f.lim, f.coef, f.vist, rec, soa, f.faceQ);
+    const bool coef = !k.coefInSweep;
+    if (k.gradient == 0) {
+        if (coef) launch_grad_lim_k<BS, true, true>(m, k, f, s, fp32, soa);
+        else launch_grad_lim_k<BS, false, true>(m, k, f, s, fp32, soa);
+    } else {
+        if (coef) launch_grad_lim_k<BS, true, false>(m, k, f, s, fp32, soa);
+        else launch_grad_lim_k<BS, false, false>(m, k, f, s, fp32, soa);
+    }
 }
 
 void launch_node_values(const DevMesh &m, DevFlow &f, hipStream_t s)
