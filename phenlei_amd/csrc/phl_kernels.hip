@@ -2342,9 +2342,11 @@ __device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, co
         }
         if (!__any(again)) break;
         // bounded wait: never reached by a correct schedule; a wave that
-        // gives up makes every later waiter give up too
-        if (wall_clock64() - t0 > waitTicks || ((it & 63) == 0 && ctl_load(&ctl[2]) != 0)) return false;
-        __builtin_amdgcn_s_sleep(1);
+        // gives up makes every later waiter give up too.  The clock is read at
+        // the first miss and every 16th after it: read every time, and a
+        // sleep with it, it sat between two polls (up to 2% of a sweep).
+        if ((it & 15) == 1 &&
+            (wall_clock64() - t0 > waitTicks || ((it & 63) == 1 && ctl_load(&ctl[2]) != 0))) return false;
     }
 #pragma unroll
     for (int s = 0; s < NW; ++s) {
@@ -2513,8 +2515,8 @@ __device__ __forceinline__ bool flow_quad(const DevMesh &M, const Consts &K, con
             again = again || wait[g];
         }
         if (!__any(again)) break;
-        if (wall_clock64() - t0 > waitTicks || ((it & 63) == 0 && ctl_load(&ctl[2]) != 0)) return false;
-        __builtin_amdgcn_s_sleep(1);
+        if ((it & 15) == 1 &&
+            (wall_clock64() - t0 > waitTicks || ((it & 63) == 1 && ctl_load(&ctl[2]) != 0))) return false;
     }
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
