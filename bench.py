@@ -712,7 +712,7 @@ def main():
                       kernel_ms=round(sweep_ms, 5), algorithmic_bytes=sb, bytes_note="496N + 96F",
                       note="latency bound: each dependency level is a launch with two dependent memory rounds"
                       if levels_form else "latency bound: one launch per direction; each dependency level costs "
-                      "a flag round trip, the neighbours' dq loads and the store acknowledgement")
+                      "one store-to-load propagation of its rows and one wavefront's arithmetic")
     print(f"[bench] mean ms per step by kernel class: {per_class}", file=sys.stderr, flush=True)
     # the dominant kernel of the step carries the contract's roofline object
     roof, other = (roof_sweep, roof_face) if sweep_ms >= flux_ms else (roof_face, roof_sweep)
