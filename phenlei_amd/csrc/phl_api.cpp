@@ -65,7 +65,6 @@ struct phl_ctx {
     // saDeferred: a relaxation is waiting for its sweeps and update.
     bool saFused = false;
     bool saDeferred = false;
-    bool sweepGaveUp = false;  // a dataflow sweep exceeded its wait bound since the last new state
     // phl_solve / phl_solve_batch: switch a mixed context to FP64 once no
     // unconverged case has halved its residual for this many steps (0: never)
     int precisionSwitchStall = 0;
@@ -378,11 +377,9 @@ phl_status check_sweep_waits(phl_ctx *c)
     int gaveUp = 0;
     HIPTRY(hipMemcpyAsync(&gaveUp, c->f.sweepCtl + 2, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPTRY(hipStreamSynchronize(c->stream));
-    if (gaveUp != 0) {
-        c->sweepGaveUp = true;
+    if (gaveUp != 0)
         return fail(PHL_ERR_NUMERIC, "dataflow sweep: " + std::to_string(gaveUp) +
                                          " wavefronts exceeded the wait bound; the state is invalid");
-    }
     return PHL_OK;
 }
 
@@ -1502,14 +1499,13 @@ phl_status phl_create_batch(const phl_mesh *pm, const phl_params *params, int de
 }
 
 // ---------------------------------------------------------------- state
-// A new state makes the context valid again after a sweep gave up waiting:
-// the count of waves that gave up is cleared with the state.
-// A new state: no sweep has given up on it.  Sweeps that did left rows of the
-// next sweep's buffer unmarked.
+// A new state makes the context valid again after a sweep gave up waiting: the
+// count of waves that gave up is cleared, and the next sweep's buffer, in
+// which such sweeps left rows unmarked, is marked again.  The count on the
+// device decides: a call may have returned on another error before it was read.
 static phl_status clear_gave_up(phl_ctx *c)
 {
-    if (c->sweepGaveUp && c->f.dqAlt) phl::launch_mark_dq(c->m, c->f.dqAlt, c->stream);
-    c->sweepGaveUp = false;
+    if (c->f.dqAlt) phl::launch_remark_dq(c->m, c->f.dqAlt, c->f.sweepCtl, c->stream);
     HIPTRY(hipMemsetAsync(c->f.sweepCtl + 2, 0, sizeof(int), c->stream));
     HIPTRY(hipStreamSynchronize(c->stream));
     return PHL_OK;

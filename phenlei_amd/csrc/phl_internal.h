@@ -313,7 +313,10 @@ void launch_dt_diag(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s
 // before the forward one, launch_sa_ghost_dq between, launch_sa_update after).
 void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool forward,
                   bool firstSweep, hipStream_t s, bool withSA = false);
+// Marks every row of a dq buffer (the next dataflow sweep's); launch_remark_dq
+// only if a wave has given up (sweepCtl[2]).
 void launch_mark_dq(const DevMesh &m, double *dq, hipStream_t s);
+void launch_remark_dq(const DevMesh &m, double *dq, const int *ctl, hipStream_t s);
 void launch_ghost_dq(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s);
 void launch_update(const DevMesh &m, const Consts &k, DevFlow &f, bool advance, hipStream_t s);
 void launch_copy(const double *src, double *dst, size_t n, hipStream_t s);

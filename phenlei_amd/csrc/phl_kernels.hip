@@ -2193,11 +2193,12 @@ __device__ __forceinline__ int ctl_load(const int *p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Both dq buffers' marks: all n values of an array.
-__global__ void __launch_bounds__(kBlock) k_mark(unsigned long long *__restrict__ a, size_t n)
+// Marks all n values of a dq buffer; with `ctl`, only if a wave has given up.
+__global__ void __launch_bounds__(kBlock) k_mark(unsigned long long *__restrict__ a, size_t n, const int *ctl)
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = kMark;
+    if (ctl && ctl[2] == 0) return;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+        a[i] = kMark;
 }
 
 // The coefficients of face side `rw` of cell cc (state qc, centroid xc, eddy
@@ -3157,13 +3158,15 @@ void launch_dt_diag(const DevMesh &m, const Consts &k, DevFlow &f, hipStream_t s
 // (barriers are cheap); larger levels are spread over the GPU.
 static const int kSmallLevel = kSweepBlock;
 
-// Marks every row of a dq buffer (the next dataflow sweep's).
-void launch_mark_dq(const DevMesh &m, double *dq, hipStream_t s)
+void launch_remark_dq(const DevMesh &m, double *dq, const int *ctl, hipStream_t s)
 {
+    // at most 2,048 workgroups, which nearly always only read the count
     const size_t n = (size_t)2 * kPlanes * m.nTotal;
-    hipLaunchKernelGGL(k_mark, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                       reinterpret_cast<unsigned long long *>(dq), n);
+    hipLaunchKernelGGL(k_mark, dim3((unsigned)std::min<size_t>((n + kBlock - 1) / kBlock, 2048)), dim3(kBlock), 0, s,
+                       reinterpret_cast<unsigned long long *>(dq), n, ctl);
 }
+
+void launch_mark_dq(const DevMesh &m, double *dq, hipStream_t s) { launch_remark_dq(m, dq, nullptr, s); }
 
 template <int NW, bool QUAD, int VIS, typename CT>
 static void launch_sweep_flow(const DevMesh &m, const Consts &k, DevFlow &f, const FlowOrder &fo, bool useU,

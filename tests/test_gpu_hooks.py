@@ -7,6 +7,8 @@ Hook order per iteration (CFD/Solver/src/Controller.cpp:567-608, 1002-1083,
 ComputeGradient, ComputeLimiter, NSSolver::UpdateResiduals (InviscidFlux,
 ViscousFlux), SpectrumRadius, TimeStep, LUSGS; then the turbulence relaxation.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -248,6 +250,35 @@ def test_sweep_wait_bound_gives_up_and_the_context_recovers(form):
     with pytest.raises(pa.PhlError) as e:
         s.lusgs()
     assert e.value.status == pa.PHL_ERR_NUMERIC
+    s.set_sweep_wait(20000000)
+    s.init_freestream()
+    ref.init_freestream()
+    assert np.array_equal(s.iterate(1, 12), ref.iterate(1, 12))
+    assert np.array_equal(s.get_state(), ref.get_state())
+
+
+@pytest.mark.parametrize("form", [0, 2, 3])
+def test_context_recovers_when_another_error_hides_that_a_sweep_gave_up(form):
+    """The same, but the call whose sweeps give up returns on a HIP error that
+    the caller's thread had pending (an impossible device, refused by the
+    runtime), before the count of waves that gave up is read: the next state
+    must not be swept with increments that were left unmarked.  With a bound of
+    20 us each direction of the 102 levels gets through its first few."""
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the instance that libphl.so is linked to
+    m = pa.Mesh.bump_hex(64, 32, 8, 0.05)
+    p = pa.default_params(mach=0.5, cfl_start=10.0, cfl_end=10.0, sweep_form=form)
+    s, ref, seen = pa.Solver(m, p), pa.Solver(m, p), pa.Solver(m, p)
+    for c in (s, seen):
+        c.init_freestream()
+        c.iterate(1, 3)  # increments of another state, to be left behind
+        c.set_sweep_wait(2000)
+    with pytest.raises(pa.PhlError) as e:
+        seen.iterate(4, 2)
+    assert e.value.status == pa.PHL_ERR_NUMERIC
+    assert hip.hipSetDevice(1 << 20) != 0
+    with pytest.raises(pa.PhlError) as e:
+        s.iterate(4, 2)
+    assert e.value.status == pa.PHL_ERR_HIP
     s.set_sweep_wait(20000000)
     s.init_freestream()
     ref.init_freestream()
