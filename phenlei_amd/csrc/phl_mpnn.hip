@@ -86,21 +86,24 @@ __global__ void __launch_bounds__(kThreads) k_input(const float *__restrict__ X,
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-// x as NP BF16 pieces.  NP 1: x rounded to nearest even.  NP 3: the exact
-// sum of three pieces (8 significant bits each, 24 in all): piece 0 is x
-// rounded, piece 1 the remainder rounded, piece 2 what is left.  That holds
-// below kSplitTop (magnitude bits), from which on x rounds to infinity.
-constexpr unsigned kSplitTop = 0x7f7f8000u;
-__device__ __forceinline__ bool splits(float x) { return (__float_as_uint(x) & 0x7fffffffu) < kSplitTop; }
+// x as NP BF16 pieces.  NP 1: x rounded to nearest even.  NP 3: three pieces
+// (8 significant bits each, 24 in all): piece 0 is x rounded, piece 1 the
+// remainder rounded, piece 2 what is left, and x is their exact sum.  It is not
+// where x rounds to infinity (from 0x7f7f8000 on, infinities and NaN among
+// them) or has bits below BF16's smallest subnormal, 2^-133 (from 2^-110 down).
+// Returns what the pieces leave of x as bits without the sign: 0 if x splits.
 template <int NP>
-__device__ __forceinline__ void split(float x, __bf16 *p)
+__device__ __forceinline__ unsigned split(float x, __bf16 *p)
 {
     p[0] = (__bf16)x;
     if constexpr (NP == 3) {
         const float r = x - (float)p[0];
         p[1] = (__bf16)r;
-        p[2] = (__bf16)(r - (float)p[1]);
+        const float s = r - (float)p[1];
+        p[2] = (__bf16)s;
+        return __float_as_uint(s - (float)p[2]) & 0x7fffffffu;
     }
+    return 0;
 }
 
 // The products of two three-piece operands that are kept beside the leading
@@ -130,9 +133,9 @@ constexpr int kTerms = 5, kTermA[kTerms] = {2, 0, 1, 1, 0}, kTermB[kTerms] = {0,
 // by the latency of a workgroup's eight chunks at two workgroups per CU.  NP 1 (inference) is bound by its 1,536 bytes of
 // activations per row: 621,818 rows in 224 us instead of 351, 4.3 TB/s.
 //
-// A value that does not split (kSplitTop; infinities and NaN among them), in
-// the rows or in the weights (`bad`, one int per workgroup of
-// k_split_weights), makes its tile be summed again value by value in FP32.
+// A value that does not split (see split), in the rows or in the weights
+// (`bad`, one int per workgroup of k_split_weights), makes its tile be summed
+// again value by value in FP32.
 constexpr int KB = 32;       // K chunk staged in LDS
 constexpr int KBP = KB + 8;  // LDS row length: 80-byte rows keep every 16-byte read aligned and conflict-free
 constexpr int kVec = TR * KB / 4 / kThreads;  // float4 of A per thread and chunk (4)
@@ -156,11 +159,11 @@ __device__ __forceinline__ void load_rows(float4 (&st)[kVec], const float *__res
     }
 }
 
-// Also the largest magnitude (as bits) of the values stored.
+// Returns nonzero if a value stored does not split.
 template <int NP>
 __device__ __forceinline__ unsigned store_rows(const float4 (&st)[kVec], __bf16 (*Al)[TR][KBP])
 {
-    unsigned top = 0;
+    unsigned left = 0;
 #pragma unroll
     for (int i = 0; i < kVec; ++i) {
         const int q = threadIdx.x + i * kThreads;
@@ -169,15 +172,14 @@ __device__ __forceinline__ unsigned store_rows(const float4 (&st)[kVec], __bf16 
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             __bf16 pc[NP];
-            split<NP>(x[e], pc);
+            left |= split<NP>(x[e], pc);
 #pragma unroll
             for (int p = 0; p < NP; ++p) v[p][e] = pc[p];
-            if constexpr (NP == 3) top = max(top, __float_as_uint(x[e]) & 0x7fffffffu);
         }
 #pragma unroll
         for (int p = 0; p < NP; ++p) *(bf16x4 *)&Al[p][q >> 3][4 * (q & 7)] = v[p];
     }
-    return top;
+    return left;
 }
 
 // The wave's weight operands of K step `step`.
@@ -221,14 +223,14 @@ __global__ void __launch_bounds__(kThreads, 2) k_dense(Product P1, Product P2, b
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     constexpr int half = H / KB;  // chunks of one operand
     const int chunks = A2 ? 2 * half : half;
-    int odd = 0;  // a value that does not split was met
+    unsigned odd = 0;  // a value that does not split was met
     if constexpr (NP == 3) odd = P1.bad[lane] | (A2 ? P2.bad[lane] : 0);
     float4 st[kVec];
     bf16x8 w[kSteps][NP][2];
     load_rows(st, A1, N, row0, 0);
 #pragma unroll
     for (int ks = 0; ks < kSteps; ++ks) load_weights<NP>(w[ks], W1, ks, wc, lane);
-    odd |= store_rows<NP>(st, Al[0]) >= kSplitTop;
+    odd |= store_rows<NP>(st, Al[0]);
     load_rows(st, A1, N, row0, KB);
     __syncthreads();
     for (int ch = 0; ch < chunks; ++ch) {
@@ -264,11 +266,11 @@ __global__ void __launch_bounds__(kThreads, 2) k_dense(Product P1, Product P2, b
             // this step's weights of the next chunk
             if (nc < chunks) load_weights<NP>(w[ks], Wn, (nc % half) * kSteps + ks, wc, lane);
         }
-        if (nc < chunks) odd |= store_rows<NP>(st, Al[nc & 1]) >= kSplitTop;
+        if (nc < chunks) odd |= store_rows<NP>(st, Al[nc & 1]);
         if (ch + 2 < chunks) load_rows(st, ch + 2 >= half ? A2 : A1, N, row0, ((ch + 2) % half) * KB);
         __syncthreads();
     }
-    if (NP == 3 && __syncthreads_or(odd)) {
+    if (NP == 3 && __syncthreads_or(odd != 0)) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -331,10 +333,10 @@ __global__ void __launch_bounds__(kThreads) k_split_weights(const float *__restr
     const int u = (int)(r / H), v = (int)(r % H);  // W[u][v] of the layer's matrix
     const float w = (((lw & 1) ? B : A) + (lw >> 1) * HH)[r];
     __bf16 p[NP];
-    split<NP>(w, p);
+    const unsigned left = split<NP>(w, p);
 #pragma unroll
     for (int q = 0; q < NP; ++q) out[(lw * NP + q) * HH + (transpose ? weight_at(v, u) : weight_at(u, v))] = p[q];
-    const int any = __syncthreads_or(!splits(w));
+    const int any = __syncthreads_or(left != 0);
     if (threadIdx.x == 0) bad[blockIdx.x] = any;
 }
 
@@ -377,7 +379,7 @@ __global__ void __launch_bounds__(kGradThreads, 2) k_wgrad_part(const float *__r
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     float st[3][8], colSum = 0.f;
-    unsigned top = 0;
+    unsigned odd = 0;
     auto load = [&](int s) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -398,11 +400,10 @@ __global__ void __launch_bounds__(kGradThreads, 2) k_wgrad_part(const float *__r
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 __bf16 p[3];
-                split<3>(st[q][i], p);
+                odd |= split<3>(st[q][i], p);
                 v[0][i] = p[0];
                 v[1][i] = p[1];
                 v[2][i] = p[2];
-                top = max(top, __float_as_uint(st[q][i]) & 0x7fffffffu);
             }
 #pragma unroll
             for (int p = 0; p < 3; ++p) *(bf16x8 *)&T[q][p][f][8 * g] = v[p];
@@ -437,7 +438,7 @@ __global__ void __launch_bounds__(kGradThreads, 2) k_wgrad_part(const float *__r
                 }
         }
     }
-    if (__syncthreads_or(top >= kSplitTop)) {  // a value that does not split: FP32 sums
+    if (__syncthreads_or(odd != 0)) {  // a value that does not split: FP32 sums
         const float *S = op ? B : A;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
