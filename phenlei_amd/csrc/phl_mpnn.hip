@@ -111,6 +111,20 @@ __device__ __forceinline__ unsigned split(float x, __bf16 *p)
 // the product, half the rounding of an FP32 product.
 constexpr int kTerms = 5, kTermA[kTerms] = {2, 0, 1, 1, 0}, kTermB[kTerms] = {0, 2, 1, 0, 1};
 
+// Nonzero if a sum of a tile is infinite or NaN.  The leading pieces are
+// rounded, so their product may overflow where that of the values does not.
+__device__ __forceinline__ unsigned not_finite(const f32x16 (&acc)[2][2])
+{
+    unsigned top = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) top = max(top, __float_as_uint(acc[i][j][r]) & 0x7fffffffu);
+    return top >= 0x7f800000u;
+}
+
 // out[N, 128] = A1[N, 128] W1 (+ A2[N, 128] W2) + bias, W1 and W2 as NP
 // pieces from k_split_weights; A split while it is staged.  Epilogue: z =
 // product + bias stored to Z (if non-null); out = z (mode 0), Hres + relu(z)
@@ -134,8 +148,8 @@ constexpr int kTerms = 5, kTermA[kTerms] = {2, 0, 1, 1, 0}, kTermB[kTerms] = {0,
 // activations per row: 621,818 rows in 224 us instead of 351, 4.3 TB/s.
 //
 // A value that does not split (see split), in the rows or in the weights
-// (`bad`, one int per workgroup of k_split_weights), makes its tile be summed
-// again value by value in FP32.
+// (`bad`, one int per workgroup of k_split_weights), or a sum that is not
+// finite, makes the tile be summed again value by value in FP32.
 constexpr int KB = 32;       // K chunk staged in LDS
 constexpr int KBP = KB + 8;  // LDS row length: 80-byte rows keep every 16-byte read aligned and conflict-free
 constexpr int kVec = TR * KB / 4 / kThreads;  // float4 of A per thread and chunk (4)
@@ -223,7 +237,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_dense(Product P1, Product P2, b
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     constexpr int half = H / KB;  // chunks of one operand
     const int chunks = A2 ? 2 * half : half;
-    unsigned odd = 0;  // a value that does not split was met
+    unsigned odd = 0;  // nonzero: the tile takes the FP32 sums
     if constexpr (NP == 3) odd = P1.bad[lane] | (A2 ? P2.bad[lane] : 0);
     float4 st[kVec];
     bf16x8 w[kSteps][NP][2];
@@ -270,6 +284,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_dense(Product P1, Product P2, b
         if (ch + 2 < chunks) load_rows(st, ch + 2 >= half ? A2 : A1, N, row0, ((ch + 2) % half) * KB);
         __syncthreads();
     }
+    if constexpr (NP == 3) odd |= not_finite(acc);
     if (NP == 3 && __syncthreads_or(odd != 0)) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -438,7 +453,8 @@ __global__ void __launch_bounds__(kGradThreads, 2) k_wgrad_part(const float *__r
                 }
         }
     }
-    if (__syncthreads_or(odd != 0)) {  // a value that does not split: FP32 sums
+    odd |= not_finite(acc);
+    if (__syncthreads_or(odd != 0)) {  // as in k_dense
         const float *S = op ? B : A;
 #pragma unroll
         for (int i = 0; i < 2; ++i)

@@ -120,3 +120,22 @@ def test_products_of_tiny_values(exponent):
                 check(gB, hv[:, None].astype(np.float64) * dz)
             if a + scale > -100:
                 check(gb0, av.astype(np.float64) * dz[0])
+
+
+@pytest.mark.parametrize("which", ["A", "B"])
+def test_products_below_the_largest_fp32(which):
+    """Products of up to 2^128 (1 - 2^-14): where the factors round up to BF16,
+    the leading pieces' product is an infinity, the values' is not."""
+    v = np.full(110, (2 - 2.0 ** -9) * 2.0 ** 63, np.float32)
+    w = np.full(5, (2 - 2.0 ** -10) * 2.0 ** 63, np.float32)
+    check(forward_products(v, w), v[:, None].astype(np.float64) * w.astype(np.float64))
+    one, small, none = (np.full(110, x, np.float32) for x in (1.0, 2.0 ** -100, 0.0))
+    dz = gradient_products(one, none, 62, which)[0]
+    v = (2.0 ** 128 * (1 - np.arange(1, 111) * 2.0 ** -14) / dz.max()).astype(np.float32)
+    dz, gA, gB, _ = gradient_products(v, none, 62, which)
+    check(gA, v[:, None].astype(np.float64) * dz)
+    check(gB, v[:, None].astype(np.float64) * dz)
+    dz = gradient_products(small, one, 62, which)[0]
+    v = (2.0 ** 128 * (1 - np.arange(1, 111) * 2.0 ** -14) / dz[0]).astype(np.float32)
+    dz, _, _, gb0 = gradient_products(small, v, 62, which)
+    check(gb0, v.astype(np.float64) * dz[0])
