@@ -107,8 +107,15 @@ __device__ __forceinline__ unsigned split(float x, __bf16 *p)
 }
 
 // The products of two three-piece operands that are kept beside the leading
-// one: piece kTermA against piece kTermB.  The dropped terms are below 2^-25 of
-// the product, half the rounding of an FP32 product.
+// one: piece kTermA against piece kTermB.  Pieces 1 and 2 are at most 2^-8 and
+// 2^-17 of a value in [1, 2), so the three left out are at most 2^-25, 2^-25 and
+// 2^-34 of a product: with the rounding of the sum a single product is within
+// 2^-23 of itself (1.78 x 2^-24 measured where every piece is as large as it can
+// be), an FP32 product within 2^-24.  The sums do not feel it: over 25 seeds each of
+// 39,600 and 123,240 rows the median error of the worst gradient tensor against
+// 64 bits was 1.2e-6 and 1.3e-6 with FP32 products, 3.0e-7 and 8.5e-7 with these
+// six terms, 3.1e-7 and 9.9e-7 with the two of 2^-25 as well, which took 5% more
+// time for a whole pass.
 constexpr int kTerms = 5, kTermA[kTerms] = {2, 0, 1, 1, 0}, kTermB[kTerms] = {0, 2, 1, 0, 1};
 
 // Nonzero if a sum of a tile is infinite or NaN.  The leading pieces are
@@ -140,11 +147,11 @@ __device__ __forceinline__ unsigned not_finite(const f32x16 (&acc)[2][2])
 //
 // NP 3 replaces v_mfma_f32_32x32x2_f32 (157 TFLOP/s): six BF16 products of
 // 16 k take 192 cycles against 512.  Its error against 64 bits is no larger:
-// network output 2.5e-7 against 2.9e-7 (200,704 rows), gradients 2.4e-7 both
-// at 315 rows and 8e-7 against 1.0e-6 at 123,240; with all six products in one
-// accumulator the gradients at 315 rows were 4% off more.  A hidden layer of
-// 200,704 rows takes 131 us instead of 262 (66 us are the bytes alone), bound
-// by the latency of a workgroup's eight chunks at two workgroups per CU.  NP 1 (inference) is bound by its 1,536 bytes of
+// network output 2.5e-7 against 2.9e-7 (200,704 rows), gradients (with
+// k_wgrad_part) 4.7e-8 against 2.4e-7 at 315 rows and as under kTerms at
+// 123,240.  A hidden layer of 200,704 rows takes 131 us instead of 262 (66 us
+// are the bytes alone), bound by the latency of a workgroup's eight chunks at
+// two workgroups per CU.  NP 1 (inference) is bound by its 1,536 bytes of
 // activations per row: 621,818 rows in 224 us instead of 351, 4.3 TB/s.
 //
 // A value that does not split (see split), in the rows or in the weights
