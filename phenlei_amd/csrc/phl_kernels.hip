@@ -2188,6 +2188,11 @@ constexpr int kRawBufferWord3 = 0x00020000;
 constexpr int kDeviceScope = 16;
 __global__ void k_sweep_ticket(int *ctl) { ctl[0] = 0; }
 
+// Between two polls of a row: the loads are plain ones to the compiler, which
+// must not take the second from the first.  (The volatile bit of the builtin's
+// cache policy would do it too, but makes the load system-scope.)
+__device__ __forceinline__ void poll_again() { __atomic_signal_fence(__ATOMIC_SEQ_CST); }
+
 __device__ __forceinline__ int ctl_load(const int *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2348,6 +2353,7 @@ __device__ __forceinline__ bool flow_chunk(const DevMesh &M, const Consts &K, co
         // sleep with it, it sat between two polls (up to 2% of a sweep).
         if ((it & 15) == 1 &&
             (wall_clock64() - t0 > waitTicks || ((it & 63) == 1 && ctl_load(&ctl[2]) != 0))) return false;
+        poll_again();
     }
 #pragma unroll
     for (int s = 0; s < NW; ++s) {
@@ -2518,6 +2524,7 @@ __device__ __forceinline__ bool flow_quad(const DevMesh &M, const Consts &K, con
         if (!__any(again)) break;
         if ((it & 15) == 1 &&
             (wall_clock64() - t0 > waitTicks || ((it & 63) == 1 && ctl_load(&ctl[2]) != 0))) return false;
+        poll_again();
     }
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
