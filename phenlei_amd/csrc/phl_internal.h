@@ -62,9 +62,11 @@ struct DevMesh {
     // the mesh's own numbering through these maps (ghost cells are not moved).
     const int *logicalOf;          // [nCell] mesh index of the cell stored at each position
     const int *cellAt;             // [nCell] storage position of each mesh cell
-    // Tile-fused face loop (kTileCells cells per workgroup): the faces touching
-    // each tile, and each cell's faces as slots of its tile's list (ELL order).
+    // Tile-fused face loop (kTileCells cells per workgroup): the cells of each
+    // tile, the faces touching them, and each cell's faces as slots of its
+    // tile's list (ELL order).
     int tileStride;                // most faces of any tile (0: the tile form is off)
+    const int *tileCells;          // [nCell] storage positions, kTileCells per tile
     const int *tileFacePtr;        // [nTiles+1]
     const int *tileFaces;          // storage face ids, ascending within a tile
     const unsigned short *c2loc;   // [W][nCell]

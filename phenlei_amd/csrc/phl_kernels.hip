@@ -1608,8 +1608,8 @@ __global__ void __launch_bounds__(BS) k_cell_gather(DevMesh M, Consts K0, const 
     }
 }
 
-// Tile-fused face loop: workgroup t owns the cells [t*BS, (t+1)*BS) of the
-// storage order.  It evaluates every face touching them (host-built list)
+// Tile-fused face loop: workgroup t owns the cells [t*BS, (t+1)*BS) of
+// tileCells.  It evaluates every face touching them (host-built list)
 // into LDS, then each thread sums its cell's faces from LDS in the cell's
 // face order, exactly like k_cell_gather sums the stored face values.  Faces
 // between two tiles are evaluated by both (identical values); the face values
@@ -1617,7 +1617,8 @@ __global__ void __launch_bounds__(BS) k_cell_gather(DevMesh M, Consts K0, const 
 template <typename T, int BS>
 __global__ void __launch_bounds__(BS) k_flux_tile(DevMesh M, Consts K0, const GatherRec *__restrict__ rec,
                                                   const T *__restrict__ gradT, const double *__restrict__ vist,
-                                                  const int *__restrict__ tileFacePtr, const int *__restrict__ tileFaces,
+                                                  const int *__restrict__ tileCells, const int *__restrict__ tileFacePtr,
+                                                  const int *__restrict__ tileFaces,
                                                   const unsigned short *__restrict__ c2loc, int ldsStride,
                                                   const double *__restrict__ q, double *__restrict__ res,
                                                   double *__restrict__ specInv, double *__restrict__ specVis,
@@ -1632,11 +1633,12 @@ __global__ void __launch_bounds__(BS) k_flux_tile(DevMesh M, Consts K0, const Ga
     for (int i = threadIdx.x; i < nf; i += BS)
         face_values<T>(M, K0, rec, gradT, vist, tileFaces[fb + i], li + (size_t)i * 6, lv + (size_t)i * 6);
     __syncthreads();
-    const int c = lb * BS + threadIdx.x;
-    const int nC = M.nCell;
+    const int nC = M.nCell, t = lb * BS + threadIdx.x;
+    const bool live = t < nC;
+    const int c = live ? tileCells[t] : 0;
     double acc[5] = {-0.0, -0.0, -0.0, -0.0, -0.0};
     double dtl = 1.0e300;
-    if (c < nC) {
+    if (live) {
         const Consts K = case_k(K0, M, c);
         double sInv = 0.0, sVis = 0.0;
         for (int s = 0; s < M.ellW; ++s) {
@@ -1681,7 +1683,7 @@ __global__ void __launch_bounds__(BS) k_flux_tile(DevMesh M, Consts K0, const Ga
     __syncthreads();  // the reduction below reuses the start of the LDS
     double *red = lds;  // [6][BS]
 #pragma unroll
-    for (int m = 0; m < 5; ++m) red[m * BS + threadIdx.x] = (c < nC) ? acc[m] * acc[m] : 0.0;
+    for (int m = 0; m < 5; ++m) red[m * BS + threadIdx.x] = live ? acc[m] * acc[m] : 0.0;
     red[5 * BS + threadIdx.x] = dtl;
     __syncthreads();
     for (int w = BS / 2; w > 0; w >>= 1) {
@@ -3047,12 +3049,14 @@ static void launch_flux_t(const DevMesh &m, const Consts &k, DevFlow &f, hipStre
         const int nb = nblk(m.nCell, kTileCells);
         if (k.mixed)
             hipLaunchKernelGGL((k_flux_tile<float, kTileCells>), dim3(nb), dim3(kTileCells), lds, s, m, k, f.rec,
-                               f.gradTF, f.vist, m.tileFacePtr, m.tileFaces, m.c2loc, m.tileStride, f.q, f.res,
-                               f.specInv, f.specVis, f.normPart, f.cflArr, f.stepCtr, f.dtLoc, f.dtMinPart, FUSED_DT);
+                               f.gradTF, f.vist, m.tileCells, m.tileFacePtr, m.tileFaces, m.c2loc, m.tileStride, f.q,
+                               f.res, f.specInv, f.specVis, f.normPart, f.cflArr, f.stepCtr, f.dtLoc, f.dtMinPart,
+                               FUSED_DT);
         else
             hipLaunchKernelGGL((k_flux_tile<double, kTileCells>), dim3(nb), dim3(kTileCells), lds, s, m, k, f.rec,
-                               f.gradT, f.vist, m.tileFacePtr, m.tileFaces, m.c2loc, m.tileStride, f.q, f.res,
-                               f.specInv, f.specVis, f.normPart, f.cflArr, f.stepCtr, f.dtLoc, f.dtMinPart, FUSED_DT);
+                               f.gradT, f.vist, m.tileCells, m.tileFacePtr, m.tileFaces, m.c2loc, m.tileStride, f.q,
+                               f.res, f.specInv, f.specVis, f.normPart, f.cflArr, f.stepCtr, f.dtLoc, f.dtMinPart,
+                               FUSED_DT);
         return;
     }
     const int nbf = nblk(m.nFace, 256);

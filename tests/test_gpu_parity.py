@@ -397,6 +397,25 @@ def test_face_loop_forms_agree(viscous):
     assert np.array_equal(a.get_residual(), b.get_residual())
 
 
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("kind,viscous", [("hex", 0), ("hex", 1), ("hybrid", 1)])
+def test_tile_fused_face_loop_runs(kind, viscous, storage):
+    """face_loop 1 is the tile form, not a silent return to the split one: the
+    sums behind the residual norm are then grouped by tiles of 128 cells, not
+    by 256 consecutive ones, so the 12 norms are not the same bits (where a
+    tile's faces do not fit the LDS, the two runs would be the same launches)."""
+    m = pa.Mesh.bump_hex(64, 32, 8, 0.05) if kind == "hex" else pa.Mesh.bump_hybrid(16, 4, 15, 1e-4, 10, 0.1, 7)
+    base = dict(mach=0.3, viscous=viscous, reynolds=5e5, cfl_start=5.0, cfl_end=5.0, storage_order=storage)
+    a = pa.Solver(m, pa.default_params(face_loop=1, **base))
+    b = pa.Solver(m, pa.default_params(face_loop=0, **base))
+    for s in (a, b):
+        s.init_freestream()
+    ha, hb = a.iterate(1, 12), b.iterate(1, 12)
+    assert not np.array_equal(ha, hb)
+    assert np.max(np.abs(ha - hb) / hb) <= 1e-14
+    assert np.array_equal(a.get_state(), b.get_state())
+
+
 @pytest.mark.parametrize("kind,precision,form", [("hex", 0, 0), ("hybrid", 0, 0), ("hybrid", 1, 0), ("wing", 0, 0),
                                                  ("hybrid", 0, 2), ("wing", 1, 2), ("hex", 0, 3), ("hybrid", 1, 3),
                                                  ("wing", 0, 3)])
