@@ -409,20 +409,28 @@ phl_status copy_field_f32(phl_ctx *c, const float *dsrc, int rows, int rowLen, i
     return copy_field_t(c, dsrc, rows, rowLen, outRowLen, out);
 }
 
-// The five components of a device array of n rows in pair planes (storage
-// order) into five host rows of outRowLen values in mesh order (zero padded).
+// Doubles of an array of n rows in the context's layout.
+size_t row_doubles(const phl_ctx *c, int n)
+{
+    return (size_t)(c->m.dqN ? 2 * phl::kPlanes : phl::kRow) * n;
+}
+
+// The five components of a device array of n rows (storage order) into five
+// host rows of outRowLen values in mesh order (zero padded).
 phl_status copy_rows(phl_ctx *c, const double *dsrc, int n, int outRowLen, double *out)
 {
     const size_t N = (size_t)n;
-    std::vector<double> h(2 * phl::kPlanes * N);
+    std::vector<double> h(row_doubles(c, n));
     if (n > 0)
         HIPTRY(hipMemcpyAsync(h.data(), dsrc, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
     HIPTRY(hipStreamSynchronize(c->stream));
     const int nC = c->m.nCell;
     for (int m = 0; m < 5; ++m) {
         double *o = out + (size_t)m * outRowLen;
-        const double *src = h.data() + (m / 2) * 2 * N + m % 2;
-        for (int i = 0; i < outRowLen; ++i) o[i] = i < n ? src[2 * (size_t)(i < nC ? c->slotOf[i] : i)] : 0.0;
+        const bool planes = c->m.dqN != 0;
+        const double *src = h.data() + (planes ? (m / 2) * 2 * N + m % 2 : m);
+        const size_t step = planes ? 2 : phl::kRow;
+        for (int i = 0; i < outRowLen; ++i) o[i] = i < n ? src[step * (size_t)(i < nC ? c->slotOf[i] : i)] : 0.0;
     }
     return PHL_OK;
 }
@@ -1298,8 +1306,11 @@ static phl_status create_impl(phl_ctx *c, const phl::Mesh &m)
         HIPTRY(hipMemset(fl.rtem, 0, sizeof(double) * nT));
     }
     k.rtem = fl.rtem;
-    TRY(dalloc(c, &fl.dq, (size_t)2 * phl::kPlanes * nT));
-    TRY(dalloc(c, &fl.dflux, (size_t)2 * phl::kPlanes * nC));
+    const bool rows = p.storage_order == 1 && c->fwd.flow.nChunks == 0 && c->bwd.flow.nChunks == 0;
+    dm.dqN = rows ? 0 : nT;
+    dm.dfluxN = rows ? 0 : nC;
+    TRY(dalloc(c, &fl.dq, row_doubles(c, nT)));
+    TRY(dalloc(c, &fl.dflux, row_doubles(c, nC)));
     fl.dqAlt = nullptr;
     fl.bwdFlow = c->bwd.flow.nChunks > 0;
     if (c->fwd.flow.nChunks > 0 || fl.bwdFlow) {
@@ -1423,8 +1434,8 @@ static phl_status create_impl(phl_ctx *c, const phl::Mesh &m)
     HIPTRY(hipMemset(fl.res, 0, sizeof(double) * 5 * nC));
     HIPTRY(hipMemset(fl.grad, 0, sizeof(double) * 15 * nC));
     HIPTRY(hipMemset(fl.gradT, 0, sizeof(double) * 3 * nC));
-    HIPTRY(hipMemset(fl.dq, 0, sizeof(double) * 2 * phl::kPlanes * nT));
-    HIPTRY(hipMemset(fl.dflux, 0, sizeof(double) * 2 * phl::kPlanes * nC));
+    HIPTRY(hipMemset(fl.dq, 0, sizeof(double) * row_doubles(c, nT)));
+    HIPTRY(hipMemset(fl.dflux, 0, sizeof(double) * row_doubles(c, nC)));
     HIPTRY(hipMemset(fl.specVis, 0, sizeof(double) * nC));
     HIPTRY(hipMemset(fl.negFlag, 0, (size_t)nC));
     HIPTRY(hipMemset(fl.negCount, 0, sizeof(int)));
@@ -1828,17 +1839,17 @@ phl_status phl_time_step(phl_ctx *c, int step)
 static void ns_sweep_pairs(phl_ctx *c, hipStream_t s)
 {
     phl::DevFlow &f = c->f;
-    const int nT = c->m.nTotal, nC = c->m.nCell;
-    hipMemsetAsync(f.dflux, 0, sizeof(double) * 2 * phl::kPlanes * nC, s);
+    const int nC = c->m.nCell;
+    hipMemsetAsync(f.dflux, 0, sizeof(double) * row_doubles(c, nC), s);
     hipMemsetAsync(f.dqPrev, 0, sizeof(double) * 5 * nC, s);
     double init = 0.0, eps = 1.1;
     c->nsLog.done = 0;
     for (int it = 0; it < c->k.nSweeps; ++it) {
         phl::launch_sweep(c->m, c->k, f, c->fwd, true, it == 0, s);
-        phl::launch_sweep_change(f.dq, nT, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm, s);
+        phl::launch_sweep_change(f.dq, c->m.dqN, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm, s);
         phl::launch_ghost_dq(c->m, c->k, f, s);
         phl::launch_sweep(c->m, c->k, f, c->bwd, false, false, s);
-        phl::launch_sweep_change(f.dq, nT, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm + 1, s);
+        phl::launch_sweep_change(f.dq, c->m.dqN, 5, nC, f.dqPrev, f.sweepParts, f.sweepNorm + 1, s);
         hipMemcpyAsync(c->nsLog.host, f.sweepNorm, 2 * sizeof(double), hipMemcpyDeviceToHost, s);
         if (hipStreamSynchronize(s) != hipSuccess) return;  // reported by the caller's launch check
         const double sn = c->nsLog.host[0] + c->nsLog.host[1];

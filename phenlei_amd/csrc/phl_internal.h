@@ -24,6 +24,20 @@ struct FaceRec {
     double lsqW;  // least-squares weight 1/(|x_R - x_L|^2 + SMALL) (gradient 1), else 0
 };
 
+// The LU-SGS increments dq and off-diagonal sums are rows of five values (a
+// sixth for the carried Spalart-Allmaras increment) in kPlanes planes of
+// 16-byte pairs, [kPlanes][rows][2]: a wavefront's access to a run of rows
+// is one contiguous 16-byte-per-lane access per plane.
+// A context whose sweeps both take the level form over cells in the mesh's
+// order has rows of kRow doubles instead, one 64-byte line each: a cell's
+// neighbours are no runs of rows there.  Level form, forward + backward per
+// step, planes against rows: mesh order 1.53 + 1.72 against 1.44 + 1.64 ms on a
+// 254k-cell hex channel and 1.16 + 1.43 against 1.12 + 1.41 on a 253k-cell
+// hybrid one; level order 1.24 + 1.36 against 1.32 + 1.39 and 1.02 + 1.26
+// against 1.08 + 1.25.
+constexpr int kPlanes = 3;
+constexpr int kRow = 8;
+
 // Read-only mesh data on the device.
 struct DevMesh {
     int nCell, nBFace, nFace, nTotal, ellW;
@@ -70,6 +84,7 @@ struct DevMesh {
     const int *tileFacePtr;        // [nTiles+1]
     const int *tileFaces;          // storage face ids, ascending within a tile
     const unsigned short *c2loc;   // [W][nCell]
+    int dqN, dfluxN;               // rows of DevFlow's dq and dflux in pair planes; 0: rows of kRow doubles
 };
 constexpr int kTileCells = 128;
 // Flagged cells of one update that SolutionFix sorts in LDS (more fall back
@@ -153,12 +168,6 @@ struct alignas(64) GatherRec {
 };
 static_assert(sizeof(GatherRec) == 192, "GatherRec is three 64-byte sectors");
 
-// The LU-SGS increments dq and off-diagonal sums are rows of five values (a
-// sixth for the carried Spalart-Allmaras increment) in kPlanes planes of
-// 16-byte pairs, [kPlanes][rows][2]: a wavefront's access to a run of rows
-// is one contiguous 16-byte-per-lane access per plane.
-constexpr int kPlanes = 3;
-
 // Mutable flow state on the device.
 struct DevFlow {
     double *q;        // [5][nTotal] primitive variables (current)
@@ -170,11 +179,11 @@ struct DevFlow {
     float *gradTF;    // [3][nCell] mixed form
     double *lim;      // [nTotal]
     double *rtem;     // [nTotal] pressure factor (entropy fix 2, 6; null otherwise)
-    double *dq;       // the increments of the last sweep: nTotal rows in pair planes (kPlanes)
+    double *dq;       // the increments of the last sweep: nTotal rows (kPlanes)
     double *dqAlt;    // dataflow sweeps: the buffer of the next sweep, every real row marked "not swept"
                       // (a sweep swaps the two; null when neither direction has a dataflow order)
     bool bwdFlow;     // the backward sweep is a dataflow sweep: ghost increments go to dqAlt
-    double *dflux;    // the off-diagonal sums of the last sweep: nCell rows in pair planes
+    double *dflux;    // the off-diagonal sums of the last sweep: nCell rows
     double *casePart; // batched contexts: [nCases][32][6] partial residual sums and dt minima
     int *sweepCtl;    // [4] dataflow sweep: ticket, unused, waves that gave up waiting, wait bound
     double *specInv, *specVis, *dtLoc, *dt, *diag;  // [nCell]
@@ -326,7 +335,7 @@ void launch_forces(const DevMesh &m, const Consts &k, DevFlow &f, const double *
 
 // Spalart-Allmaras (phl_sa.hip).  tri: [nTri][9] wall triangles (face centre
 // and two consecutive face nodes).
-// nv 5: dq in pair planes of n rows; nv 1: a plain array.
+// nv 5: dq in pair planes of n rows (0: rows of kRow doubles); nv 1: a plain array.
 void launch_sweep_change(const double *dq, int n, int nv, int nC, double *prev, double *parts, double *out,
                          hipStream_t s);
 void launch_wall_distance(const double *xcc, const double *ycc, const double *zcc, int nCell, const double *tri,

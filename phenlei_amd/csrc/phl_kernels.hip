@@ -268,6 +268,35 @@ __device__ __forceinline__ void store_row5(double *a, int n, int i, const double
     pair_at(a, n, i, 2)->x = v[4];
 }
 
+// The same in rows of kRow doubles, and in the layout that the context chose: n
+// 0 for rows of kRow, else pair planes of n rows.
+__device__ __forceinline__ void load_line5(const double *a, int i, double *v)
+{
+    const double2 *p = reinterpret_cast<const double2 *>(a) + (size_t)i * (kRow / 2);
+    const double2 x = p[0], y = p[1];
+    v[0] = x.x; v[1] = x.y; v[2] = y.x; v[3] = y.y; v[4] = p[2].x;
+}
+
+__device__ __forceinline__ void store_line5(double *a, int i, const double *v)
+{
+    double2 *p = reinterpret_cast<double2 *>(a) + (size_t)i * (kRow / 2);
+    p[0] = make_double2(v[0], v[1]);
+    p[1] = make_double2(v[2], v[3]);
+    p[2].x = v[4];
+}
+
+__device__ __forceinline__ void load_any5(const double *a, int n, int i, double *v)
+{
+    if (n) load_row5(a, n, i, v);
+    else load_line5(a, i, v);
+}
+
+__device__ __forceinline__ void store_any5(double *a, int n, int i, const double *v)
+{
+    if (n) store_row5(a, n, i, v);
+    else store_line5(a, i, v);
+}
+
 // The "not swept yet" mark of an increment (all bits set, a NaN that no
 // arithmetic of the hardware produces), and a value made distinct from it (a
 // NaN payload carried in from the caller's state).
@@ -1755,8 +1784,8 @@ __global__ void __launch_bounds__(kBlock) k_norm_sum5(const double *__restrict__
 // The squared change of dq since the last call (the sweepNormal of
 // Controller::LUSGS for nLUSGSSweeps > 1, Controller.cpp:1920-1950; the
 // reference adds SQR(dq - dqOld) cell by cell in its sweeps): per block of
-// kBlock real cells, over nv components (5: pair planes of n rows; 1: a plain
-// array), and prev [nv][nC] takes the new dq.  k_sum_into then adds the block
+// kBlock real cells, over nv components (5: rows as load_any5 has them; 1: a
+// plain array), and prev [nv][nC] takes the new dq.  k_sum_into then adds the block
 // partials in a fixed order.
 __global__ void __launch_bounds__(kBlock) k_sweep_change(const double *__restrict__ dq, int n, int nv, int nC,
                                                          double *__restrict__ prev, double *__restrict__ parts)
@@ -1766,7 +1795,7 @@ __global__ void __launch_bounds__(kBlock) k_sweep_change(const double *__restric
     double acc = 0.0;
     if (c < nC) {
         double v[5];
-        if (nv == 5) load_row5(dq, n, c, v);
+        if (nv == 5) load_any5(dq, n, c, v);
         else v[0] = dq[c];
         for (int m = 0; m < nv; ++m) {
             const double d = v[m] - prev[(size_t)m * nC + c];
@@ -1925,15 +1954,15 @@ __device__ __forceinline__ void sweep_finish(const DevMesh &M, int c, bool useU,
     double r[5], U[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     load5(res, nC, c, r);
     const double D = diag[c];
-    if (useU) load_row5(dflux, M.nCell, c, U);
+    if (useU) load_any5(dflux, M.dfluxN, c, U);
     double v[5], w[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         v[m] = (r[m] - U[m] - rhs0[m]) / D;
         w[m] = 0.0 + rhs0[m];
     }
-    store_row5(dq, M.nTotal, c, v);
-    store_row5(dflux, M.nCell, c, w);
+    store_any5(dq, M.dqN, c, v);
+    store_any5(dflux, M.dfluxN, c, w);
 }
 
 __device__ __forceinline__ void load_coef(const double *__restrict__ coef, int f, bool isL, double *co)
@@ -1977,7 +2006,7 @@ __device__ __forceinline__ void sweep_cell_batched(const DevMesh &M, const Const
         const bool isL = enc[s] > 0;
         const int f = act[s] ? (isL ? enc[s] : -enc[s]) - 1 : 0;
         load_coef(coef, f, isL, co[s]);
-        load_row5(dq, M.nTotal, act[s] ? nb[s] : 0, dqn[s]);
+        load_any5(dq, M.dqN, act[s] ? nb[s] : 0, dqn[s]);
     }
     double rhs0[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -2008,7 +2037,7 @@ __device__ __forceinline__ void sweep_cell_generic(const DevMesh &M, const Const
         const int f = (isL ? enc : -enc) - 1;
         double co[15], dqn[5], df[5];
         load_coef(coef, f, isL, co);
-        load_row5(dq, M.nTotal, nb, dqn);
+        load_any5(dq, M.dqN, nb, dqn);
         sweep_apply(K, co, dqn, df);
 #pragma unroll
         for (int m = 0; m < 5; ++m) rhs0[m] += df[m];
@@ -2079,7 +2108,8 @@ __device__ __forceinline__ void load_coef_row(const double *__restrict__ coef, i
     }
 }
 
-template <int NW, int VIS, typename CT>
+// LINES: the increments are rows of kRow doubles.
+template <int NW, int VIS, typename CT, bool LINES>
 __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K, const SweepOrder &so, int p,
                                                bool useU, const double *__restrict__ coef,
                                                const double *__restrict__ res, const double *__restrict__ diag,
@@ -2097,13 +2127,17 @@ __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K
     double r[5], U[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     load5(res, P, c, r);
     const double D = diag[c];
-    if (useU) load_row5(dflux, M.nCell, c, U);
+    if (useU) {
+        if constexpr (LINES) load_line5(dflux, c, U);
+        else load_row5(dflux, P, c, U);
+    }
     double co[NW][16], dqn[NW][5];
 #pragma unroll
     for (int s = 0; s < NW; ++s) {
         const bool act = row[s] >= 0;
         load_coef_row<CT>(coef, act ? row[s] : 0, co[s]);
-        load_row5(dq, M.nTotal, act ? nb[s] : 0, dqn[s]);
+        if constexpr (LINES) load_line5(dq, act ? nb[s] : 0, dqn[s]);
+        else load_row5(dq, M.nTotal, act ? nb[s] : 0, dqn[s]);
     }
     // Unused slots add +0.0, which leaves the sum unchanged (it starts at
     // +0.0, so it is never -0.0); no branch lets the loads of a slot sink.
@@ -2122,21 +2156,26 @@ __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K
         v[m] = (r[m] - U[m] - rhs0[m]) / D;
         w[m] = 0.0 + rhs0[m];
     }
-    store_row5(dq, M.nTotal, c, v);
-    store_row5(dflux, M.nCell, c, w);
+    if constexpr (LINES) {
+        store_line5(dq, c, v);
+        store_line5(dflux, c, w);
+    } else {
+        store_row5(dq, M.nTotal, c, v);
+        store_row5(dflux, P, c, w);
+    }
 }
 
-template <int NW, int VIS, typename CT>
+template <int NW, int VIS, typename CT, bool LINES>
 __global__ void __launch_bounds__(64) k_sweep_level_so(DevMesh M, Consts K, SweepOrder so, int begin, int end,
                                                        bool useU, const double *__restrict__ coef,
                                                        const double *__restrict__ res, const double *__restrict__ diag, double *dq, double *dflux)
 {
     const int p = begin + xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (p >= end) return;
-    sweep_position<NW, VIS, CT>(M, K, so, p, useU, coef, res, diag, dq, dflux);
+    sweep_position<NW, VIS, CT, LINES>(M, K, so, p, useU, coef, res, diag, dq, dflux);
 }
 
-template <int NW, int VIS, typename CT>
+template <int NW, int VIS, typename CT, bool LINES>
 __global__ void __launch_bounds__(kSweepBlock) k_sweep_block_so(DevMesh M, Consts K, SweepOrder so,
                                                                const int *__restrict__ ptr, int l0, int l1,
                                                                bool useU, const double *__restrict__ coef,
@@ -2146,7 +2185,7 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_block_so(DevMesh M, Const
     for (int L = l0; L < l1; ++L) {
         const int b = ptr[L], e = ptr[L + 1];
         for (int p = b + (int)threadIdx.x; p < e; p += blockDim.x)
-            sweep_position<NW, VIS, CT>(M, K, so, p, useU, coef, res, diag, dq, dflux);
+            sweep_position<NW, VIS, CT, LINES>(M, K, so, p, useU, coef, res, diag, dq, dflux);
         __syncthreads();
     }
 }
@@ -2620,7 +2659,7 @@ __global__ void __launch_bounds__(kBlock) k_ghost_dq(DevMesh M, Consts K, const 
     const int le = M.fle[f], re = M.nCell + f;
     const int bc = M.bcType[f];
     double dl[5], dr[5];
-    load_row5(dq, nT, le, dl);
+    load_any5(dq, M.dqN, le, dl);
     if (bc == kBC_SYMM || (bc == kBC_WALL && !K.viscous)) {
         double prim[5], Q[5];
         load5(q, nT, le, prim);
@@ -2661,7 +2700,7 @@ __global__ void __launch_bounds__(kBlock) k_ghost_dq(DevMesh M, Consts K, const 
     }
 #pragma unroll
     for (int m = 0; m < 5; ++m) dr[m] = not_mark(dr[m]);
-    store_row5(out, nT, re, dr);
+    store_any5(out, M.dqN, re, dr);
 }
 
 // ------------------------------------------------------------- update
@@ -2686,7 +2725,7 @@ __global__ void __launch_bounds__(kBlock) k_update(DevMesh M, Consts K0, const d
         Q[0] = prim[0]; Q[1] = prim[0] * prim[1]; Q[2] = prim[0] * prim[2]; Q[3] = prim[0] * prim[3];
         Q[4] = prim[0] * em;
         double d5[5];
-        load_row5(dq, nT, i, d5);
+        load_any5(dq, M.dqN, i, d5);
 #pragma unroll
         for (int m = 0; m < 5; ++m) Q[m] += d5[m];
         if (Q[0] <= 0.0) {
@@ -3210,9 +3249,9 @@ static void launch_sweep_flow_w(const DevMesh &m, const Consts &k, DevFlow &f, c
     }
 }
 
-template <int NW, int VIS, typename CT>
-static void launch_sweep_so(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool useU,
-                            hipStream_t s)
+template <int NW, int VIS, typename CT, bool LINES>
+static void launch_sweep_levels(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool useU,
+                                hipStream_t s)
 {
     int L = 0;
     while (L < lv.nLevels) {
@@ -3220,15 +3259,23 @@ static void launch_sweep_so(const DevMesh &m, const Consts &k, DevFlow &f, const
         if (sz <= kSmallLevel) {
             int L1 = L + 1;
             while (L1 < lv.nLevels && lv.hptr[L1 + 1] - lv.hptr[L1] <= kSmallLevel) ++L1;
-            hipLaunchKernelGGL((k_sweep_block_so<NW, VIS, CT>), dim3(1), dim3(kSweepBlock), 0, s, m, k, lv.so, lv.ptr, L,
-                               L1, useU, f.coef, f.res, f.diag, f.dq, f.dflux);
+            hipLaunchKernelGGL((k_sweep_block_so<NW, VIS, CT, LINES>), dim3(1), dim3(kSweepBlock), 0, s, m, k, lv.so,
+                               lv.ptr, L, L1, useU, f.coef, f.res, f.diag, f.dq, f.dflux);
             L = L1;
         } else {
-            hipLaunchKernelGGL((k_sweep_level_so<NW, VIS, CT>), dim3(nblk(sz, 64)), dim3(64), 0, s, m, k, lv.so,
+            hipLaunchKernelGGL((k_sweep_level_so<NW, VIS, CT, LINES>), dim3(nblk(sz, 64)), dim3(64), 0, s, m, k, lv.so,
                                lv.hptr[L], lv.hptr[L + 1], useU, f.coef, f.res, f.diag, f.dq, f.dflux);
             ++L;
         }
     }
+}
+
+template <int NW, int VIS, typename CT>
+static void launch_sweep_so(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool useU,
+                            hipStream_t s)
+{
+    if (m.dqN == 0) launch_sweep_levels<NW, VIS, CT, true>(m, k, f, lv, useU, s);
+    else launch_sweep_levels<NW, VIS, CT, false>(m, k, f, lv, useU, s);
 }
 
 void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool forward,

@@ -795,7 +795,8 @@ __global__ void __launch_bounds__(kBlock) k_sa_ghost_dq(DevMesh M, double *__res
     const bool copy = bc == kBC_FAR || bc == kBC_SYMM || bc == kBC_INFLOW || bc == kBC_OUTFLOW;
     const double v = copy ? dq[M.fle[f]] : 0.0;
     dq[M.nCell + f] = v;
-    rows[((size_t)(kPlanes - 1) * M.nTotal + M.nCell + f) * 2 + 1] = v;  // the sixth value of the ghost's dq row
+    // the sixth value of the ghost's dq row, for a sweep that carries this one
+    if (M.dqN) rows[((size_t)(kPlanes - 1) * M.nTotal + M.nCell + f) * 2 + 1] = v;
 }
 
 __global__ void __launch_bounds__(kBlock) k_sa_update(DevMesh M, double *__restrict__ nut,
