@@ -268,8 +268,9 @@ __device__ __forceinline__ void store_row5(double *a, int n, int i, const double
     pair_at(a, n, i, 2)->x = v[4];
 }
 
-// The same in rows of kRow doubles, and in the layout that the context chose: n
-// 0 for rows of kRow, else pair planes of n rows.
+// The same in rows of kRow doubles; in either layout, LINES for those; and in the
+// layout that the context chose, n 0 for them (a test that costs the level
+// kernels 6% where it is not settled when they are compiled).
 __device__ __forceinline__ void load_line5(const double *a, int i, double *v)
 {
     const double2 *p = reinterpret_cast<const double2 *>(a) + (size_t)i * (kRow / 2);
@@ -283,6 +284,20 @@ __device__ __forceinline__ void store_line5(double *a, int i, const double *v)
     p[0] = make_double2(v[0], v[1]);
     p[1] = make_double2(v[2], v[3]);
     p[2].x = v[4];
+}
+
+template <bool LINES>
+__device__ __forceinline__ void load_inc(const double *a, int n, int i, double *v)
+{
+    if constexpr (LINES) load_line5(a, i, v);
+    else load_row5(a, n, i, v);
+}
+
+template <bool LINES>
+__device__ __forceinline__ void store_inc(double *a, int n, int i, const double *v)
+{
+    if constexpr (LINES) store_line5(a, i, v);
+    else store_row5(a, n, i, v);
 }
 
 __device__ __forceinline__ void load_any5(const double *a, int n, int i, double *v)
@@ -1945,6 +1960,7 @@ __global__ void __launch_bounds__(kBlock) k_dt_diag(DevMesh M, Consts K, const d
     diag[c] = D;
 }
 
+template <bool LINES>
 __device__ __forceinline__ void sweep_finish(const DevMesh &M, int c, bool useU, const double *rhs0,
                                              const double *__restrict__ res, const double *__restrict__ diag,
                                              double *dq, double *dflux)
@@ -1954,15 +1970,15 @@ __device__ __forceinline__ void sweep_finish(const DevMesh &M, int c, bool useU,
     double r[5], U[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     load5(res, nC, c, r);
     const double D = diag[c];
-    if (useU) load_any5(dflux, M.dfluxN, c, U);
+    if (useU) load_inc<LINES>(dflux, nC, c, U);
     double v[5], w[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         v[m] = (r[m] - U[m] - rhs0[m]) / D;
         w[m] = 0.0 + rhs0[m];
     }
-    store_any5(dq, M.dqN, c, v);
-    store_any5(dflux, M.dfluxN, c, w);
+    store_inc<LINES>(dq, M.nTotal, c, v);
+    store_inc<LINES>(dflux, nC, c, w);
 }
 
 __device__ __forceinline__ void load_coef(const double *__restrict__ coef, int f, bool isL, double *co)
@@ -1983,7 +1999,7 @@ __device__ __forceinline__ void load_coef(const double *__restrict__ coef, int f
 // so a level costs a few memory latencies.
 constexpr int kW = 6;
 constexpr int kSweepBlock = 512;
-template <bool FWD>
+template <bool FWD, bool LINES>
 __device__ __forceinline__ void sweep_cell_batched(const DevMesh &M, const Consts &K, int c, bool useU,
                                                    const double *__restrict__ coef, const double *__restrict__ res, const double *__restrict__ diag,
                                                    double *dq, double *dflux)
@@ -2006,7 +2022,7 @@ __device__ __forceinline__ void sweep_cell_batched(const DevMesh &M, const Const
         const bool isL = enc[s] > 0;
         const int f = act[s] ? (isL ? enc[s] : -enc[s]) - 1 : 0;
         load_coef(coef, f, isL, co[s]);
-        load_any5(dq, M.dqN, act[s] ? nb[s] : 0, dqn[s]);
+        load_inc<LINES>(dq, M.nTotal, act[s] ? nb[s] : 0, dqn[s]);
     }
     double rhs0[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -2017,11 +2033,11 @@ __device__ __forceinline__ void sweep_cell_batched(const DevMesh &M, const Const
 #pragma unroll
         for (int m = 0; m < 5; ++m) rhs0[m] += df[m];
     }
-    sweep_finish(M, c, useU, rhs0, res, diag, dq, dflux);
+    sweep_finish<LINES>(M, c, useU, rhs0, res, diag, dq, dflux);
 }
 
 // Any number of faces per cell (polyhedral meshes): face by face.
-template <bool FWD>
+template <bool FWD, bool LINES>
 __device__ __forceinline__ void sweep_cell_generic(const DevMesh &M, const Consts &K, int c, bool useU,
                                                    const double *__restrict__ coef, const double *__restrict__ res, const double *__restrict__ diag,
                                                    double *dq, double *dflux)
@@ -2037,24 +2053,24 @@ __device__ __forceinline__ void sweep_cell_generic(const DevMesh &M, const Const
         const int f = (isL ? enc : -enc) - 1;
         double co[15], dqn[5], df[5];
         load_coef(coef, f, isL, co);
-        load_any5(dq, M.dqN, nb, dqn);
+        load_inc<LINES>(dq, M.nTotal, nb, dqn);
         sweep_apply(K, co, dqn, df);
 #pragma unroll
         for (int m = 0; m < 5; ++m) rhs0[m] += df[m];
     }
-    sweep_finish(M, c, useU, rhs0, res, diag, dq, dflux);
+    sweep_finish<LINES>(M, c, useU, rhs0, res, diag, dq, dflux);
 }
 
-template <bool FWD>
+template <bool FWD, bool LINES>
 __device__ __forceinline__ void sweep_cell(const DevMesh &M, const Consts &K, int c, bool useU,
                                            const double *__restrict__ coef, const double *__restrict__ res, const double *__restrict__ diag, double *dq, double *dflux)
 {
-    if (M.ellW <= kW) sweep_cell_batched<FWD>(M, K, c, useU, coef, res, diag, dq, dflux);
-    else sweep_cell_generic<FWD>(M, K, c, useU, coef, res, diag, dq, dflux);
+    if (M.ellW <= kW) sweep_cell_batched<FWD, LINES>(M, K, c, useU, coef, res, diag, dq, dflux);
+    else sweep_cell_generic<FWD, LINES>(M, K, c, useU, coef, res, diag, dq, dflux);
 }
 
 // One level spread over the whole GPU (64-thread workgroups).
-template <bool FWD>
+template <bool FWD, bool LINES>
 __global__ void __launch_bounds__(64) k_sweep_level(DevMesh M, Consts K, const int *__restrict__ cells, int begin,
                                                     int end, bool useU, const double *__restrict__ coef,
                                                     const double *__restrict__ res, const double *__restrict__ diag,
@@ -2062,12 +2078,12 @@ __global__ void __launch_bounds__(64) k_sweep_level(DevMesh M, Consts K, const i
 {
     const int i = begin + xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (i >= end) return;
-    sweep_cell<FWD>(M, K, cells[i], useU, coef, res, diag, dq, dflux);
+    sweep_cell<FWD, LINES>(M, K, cells[i], useU, coef, res, diag, dq, dflux);
 }
 
 // One workgroup walks a run of small levels; the barrier between levels
 // makes the previous level's dq visible to the whole workgroup.
-template <bool FWD>
+template <bool FWD, bool LINES>
 __global__ void __launch_bounds__(kSweepBlock) k_sweep_block(DevMesh M, Consts K, const int *__restrict__ ptr,
                                                       const int *__restrict__ cells, int l0, int l1, bool useU,
                                                       const double *__restrict__ coef, const double *__restrict__ res, const double *__restrict__ diag, double *dq, double *dflux)
@@ -2075,7 +2091,7 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_block(DevMesh M, Consts K
     for (int L = l0; L < l1; ++L) {
         const int b = ptr[L], e = ptr[L + 1];
         for (int i = b + (int)threadIdx.x; i < e; i += blockDim.x)
-            sweep_cell<FWD>(M, K, cells[i], useU, coef, res, diag, dq, dflux);
+            sweep_cell<FWD, LINES>(M, K, cells[i], useU, coef, res, diag, dq, dflux);
         __syncthreads();
     }
 }
@@ -2108,7 +2124,6 @@ __device__ __forceinline__ void load_coef_row(const double *__restrict__ coef, i
     }
 }
 
-// LINES: the increments are rows of kRow doubles.
 template <int NW, int VIS, typename CT, bool LINES>
 __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K, const SweepOrder &so, int p,
                                                bool useU, const double *__restrict__ coef,
@@ -2127,17 +2142,13 @@ __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K
     double r[5], U[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     load5(res, P, c, r);
     const double D = diag[c];
-    if (useU) {
-        if constexpr (LINES) load_line5(dflux, c, U);
-        else load_row5(dflux, P, c, U);
-    }
+    if (useU) load_inc<LINES>(dflux, P, c, U);
     double co[NW][16], dqn[NW][5];
 #pragma unroll
     for (int s = 0; s < NW; ++s) {
         const bool act = row[s] >= 0;
         load_coef_row<CT>(coef, act ? row[s] : 0, co[s]);
-        if constexpr (LINES) load_line5(dq, act ? nb[s] : 0, dqn[s]);
-        else load_row5(dq, M.nTotal, act ? nb[s] : 0, dqn[s]);
+        load_inc<LINES>(dq, M.nTotal, act ? nb[s] : 0, dqn[s]);
     }
     // Unused slots add +0.0, which leaves the sum unchanged (it starts at
     // +0.0, so it is never -0.0); no branch lets the loads of a slot sink.
@@ -2156,13 +2167,8 @@ __device__ __forceinline__ void sweep_position(const DevMesh &M, const Consts &K
         v[m] = (r[m] - U[m] - rhs0[m]) / D;
         w[m] = 0.0 + rhs0[m];
     }
-    if constexpr (LINES) {
-        store_line5(dq, c, v);
-        store_line5(dflux, c, w);
-    } else {
-        store_row5(dq, M.nTotal, c, v);
-        store_row5(dflux, P, c, w);
-    }
+    store_inc<LINES>(dq, M.nTotal, c, v);
+    store_inc<LINES>(dflux, P, c, w);
 }
 
 template <int NW, int VIS, typename CT, bool LINES>
@@ -3278,6 +3284,28 @@ static void launch_sweep_so(const DevMesh &m, const Consts &k, DevFlow &f, const
     else launch_sweep_levels<NW, VIS, CT, false>(m, k, f, lv, useU, s);
 }
 
+// Wider polyhedra: face by face through the cell -> face lists.
+template <bool FWD, bool LINES>
+static void launch_sweep_lists(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool useU,
+                               hipStream_t s)
+{
+    int L = 0;
+    while (L < lv.nLevels) {
+        const int sz = lv.hptr[L + 1] - lv.hptr[L];
+        if (sz <= kSmallLevel) {
+            int L1 = L + 1;
+            while (L1 < lv.nLevels && lv.hptr[L1 + 1] - lv.hptr[L1] <= kSmallLevel) ++L1;
+            hipLaunchKernelGGL((k_sweep_block<FWD, LINES>), dim3(1), dim3(kSweepBlock), 0, s, m, k, lv.ptr, lv.cells, L,
+                               L1, useU, f.coef, f.res, f.diag, f.dq, f.dflux);
+            L = L1;
+        } else {
+            hipLaunchKernelGGL((k_sweep_level<FWD, LINES>), dim3(nblk(sz, 64)), dim3(64), 0, s, m, k, lv.cells,
+                               lv.hptr[L], lv.hptr[L + 1], useU, f.coef, f.res, f.diag, f.dq, f.dflux);
+            ++L;
+        }
+    }
+}
+
 void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &lv, bool forward,
                   bool firstSweep, hipStream_t s, bool withSA)
 {
@@ -3301,29 +3329,12 @@ void launch_sweep(const DevMesh &m, const Consts &k, DevFlow &f, const Levels &l
     if (lv.so.Wpad == 3) return v ? launch_sweep_so<3, 1, double>(m, k, f, lv, useU, s) : launch_sweep_so<3, 0, double>(m, k, f, lv, useU, s);
     if (lv.so.Wpad == 4) return v ? launch_sweep_so<4, 1, double>(m, k, f, lv, useU, s) : launch_sweep_so<4, 0, double>(m, k, f, lv, useU, s);
     if (lv.so.Wpad == 6) return v ? launch_sweep_so<6, 1, double>(m, k, f, lv, useU, s) : launch_sweep_so<6, 0, double>(m, k, f, lv, useU, s);
-    // wider polyhedra: face-by-face through the cell -> face lists
-    int L = 0;
-    while (L < lv.nLevels) {
-        const int sz = lv.hptr[L + 1] - lv.hptr[L];
-        if (sz <= kSmallLevel) {
-            int L1 = L + 1;
-            while (L1 < lv.nLevels && lv.hptr[L1 + 1] - lv.hptr[L1] <= kSmallLevel) ++L1;
-            if (forward)
-                hipLaunchKernelGGL(k_sweep_block<true>, dim3(1), dim3(kSweepBlock), 0, s, m, k, lv.ptr, lv.cells, L, L1,
-                                   useU, f.coef, f.res, f.diag, f.dq, f.dflux);
-            else
-                hipLaunchKernelGGL(k_sweep_block<false>, dim3(1), dim3(kSweepBlock), 0, s, m, k, lv.ptr, lv.cells, L, L1,
-                                   useU, f.coef, f.res, f.diag, f.dq, f.dflux);
-            L = L1;
-        } else {
-            if (forward)
-                hipLaunchKernelGGL(k_sweep_level<true>, dim3(nblk(sz, 64)), dim3(64), 0, s, m, k, lv.cells,
-                                   lv.hptr[L], lv.hptr[L + 1], useU, f.coef, f.res, f.diag, f.dq, f.dflux);
-            else
-                hipLaunchKernelGGL(k_sweep_level<false>, dim3(nblk(sz, 64)), dim3(64), 0, s, m, k, lv.cells,
-                                   lv.hptr[L], lv.hptr[L + 1], useU, f.coef, f.res, f.diag, f.dq, f.dflux);
-            ++L;
-        }
+    if (m.dqN == 0) {
+        if (forward) launch_sweep_lists<true, true>(m, k, f, lv, useU, s);
+        else launch_sweep_lists<false, true>(m, k, f, lv, useU, s);
+    } else {
+        if (forward) launch_sweep_lists<true, false>(m, k, f, lv, useU, s);
+        else launch_sweep_lists<false, false>(m, k, f, lv, useU, s);
     }
 }
 

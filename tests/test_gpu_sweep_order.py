@@ -142,3 +142,11 @@ def test_one_direction_in_dataflow_form_the_other_by_level(wide_first):
     a, b = run(mesh, 5, sweep_form=0), run(mesh, 5, sweep_form=1)
     for k in a:
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("wide_first", [True, False])
+def test_level_form_of_wide_cells_in_mesh_order(wide_first):
+    mesh = wide_cell_mesh(wide_first)
+    a, b = run(mesh, 5, sweep_form=1, storage_order=1), run(mesh, 5, sweep_form=1)
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
