@@ -50,10 +50,11 @@ struct phl_ctx {
     std::vector<hipEvent_t> events;
     double kernelMs[PHL_N_KERNEL_CLASSES] = {0};
     int timedSteps = 0;
-    // hipGraphs of kGraphSteps steps, one per assignment of the q / qAlt buffers
+    // hipGraphs of kGraphSteps steps, one per assignment of the q / qAlt and the
+    // dq / dqAlt buffers, whose addresses they hold
     int launchMode = 1;  // 0 eager, 1 graph, 2 eager with the turbulence sweeps on the side stream
-    double *qBuf0 = nullptr;
-    hipGraphExec_t stepGraph[2] = {nullptr, nullptr};
+    double *qBuf0 = nullptr, *dqBuf0 = nullptr;
+    hipGraphExec_t stepGraph[4] = {nullptr, nullptr, nullptr, nullptr};
     // Spalart-Allmaras: the scalar sweeps of a step touch only nu~ and the
     // turbulence LU-SGS arrays, which the next step's NS kernels do not use,
     // so they run on `side` beside them; evJoin orders the next relaxation
@@ -1310,6 +1311,7 @@ static phl_status create_impl(phl_ctx *c, const phl::Mesh &m)
     dm.dqN = rows ? 0 : nT;
     dm.dfluxN = rows ? 0 : nC;
     TRY(dalloc(c, &fl.dq, row_doubles(c, nT)));
+    c->dqBuf0 = fl.dq;
     TRY(dalloc(c, &fl.dflux, row_doubles(c, nC)));
     fl.dqAlt = nullptr;
     fl.bwdFlow = c->bwd.flow.nChunks > 0;
@@ -2151,30 +2153,32 @@ static void enqueue_step(phl_ctx *c, hipEvent_t *ev)
 }
 
 // kGraphSteps consecutive steps captured as one hipGraph.  A step swaps q
-// and qAlt, so after an even number of steps the buffers are back where they
-// started and the graph can be replayed; one graph is kept for each
-// assignment of the buffers.  The captured sequence holds kernels and the
+// and qAlt, and dq and dqAlt once for each direction in dataflow form, so after
+// an even number of steps the buffers are back where they started and the
+// graph can be replayed; one graph is kept for each assignment of the buffers.
+// The captured sequence holds kernels and the
 // event edges between the solver and side streams; it starts and ends with
 // the side stream joined.
 static const int kGraphSteps = 8;
 static phl_status step_graph(phl_ctx *c, hipGraphExec_t *out)
 {
-    const int parity = c->f.q == c->qBuf0 ? 0 : 1;
-    if (!c->stepGraph[parity]) {
+    static_assert(kGraphSteps % 2 == 0, "the buffers are back after a replay");
+    const int which = (c->f.q == c->qBuf0 ? 0 : 1) + (c->f.dq == c->dqBuf0 ? 0 : 2);
+    if (!c->stepGraph[which]) {
         hipGraph_t g = nullptr;
         HIPTRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         for (int i = 0; i < kGraphSteps; ++i) enqueue_step(c, nullptr);
         join_turb(c);
         HIPTRY(hipStreamEndCapture(c->stream, &g));
-        const hipError_t e = hipGraphInstantiate(&c->stepGraph[parity], g, nullptr, nullptr, 0);
+        const hipError_t e = hipGraphInstantiate(&c->stepGraph[which], g, nullptr, nullptr, 0);
         hipGraphDestroy(g);
         if (e != hipSuccess) {
-            c->stepGraph[parity] = nullptr;
+            c->stepGraph[which] = nullptr;
             return fail(PHL_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
         }
         // capturing swapped the buffers kGraphSteps times: back at the start
     }
-    *out = c->stepGraph[parity];
+    *out = c->stepGraph[which];
     return PHL_OK;
 }
 

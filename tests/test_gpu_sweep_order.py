@@ -150,3 +150,30 @@ def test_level_form_of_wide_cells_in_mesh_order(wide_first):
     a, b = run(mesh, 5, sweep_form=1, storage_order=1), run(mesh, 5, sweep_form=1)
     for k in a:
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("wide_first", [True, False])
+def test_graphs_with_one_direction_in_dataflow_form(wide_first):
+    """A step then swaps the two increment buffers once, so that eight-step
+    graphs start from either assignment: replays after odd numbers of steps
+    and after a hook's sweep equal eager launches of the level form."""
+    mesh = wide_cell_mesh(wide_first)
+    p = [pa.default_params(mach=0.5, cfl_start=2.0, cfl_end=2.0, viscous=1, reynolds=5e4, sweep_form=f) for f in (0, 1)]
+    a, b = (pa.Solver(mesh, q) for q in p)
+    b.set_launch_mode("eager")
+    step = 1
+    for s in (a, b):
+        s.init_freestream()
+        s.set_state(perturbed_state(mesh.n_total, mesh.n_cell, FREE, 5, amp=0.01))
+    for n in (8, 3, 17, 1, 24):
+        assert np.array_equal(a.iterate(step, n), b.iterate(step, n)), n
+        step += n
+        for s in (a, b):
+            s.residual()
+            s.spectrum_radius()
+            s.time_step(step)
+            s.lusgs()
+        step += 1
+        for k in ("q", "res", "dq", "delta_flux"):
+            assert np.array_equal(a.get_field(k), b.get_field(k)), (n, k)
+    assert a.launch_counts()[0] >= 6
