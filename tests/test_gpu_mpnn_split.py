@@ -82,3 +82,45 @@ def test_values_that_do_not_split(where, value):
         z = h @ p["A"][0] + m @ p["B"][0]
         want = (h + relu(z)) @ p["Wo"]
     assert np.array_equal(net.forward(), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("n,layers", [(8193, 6), (20011, 6), (70001, 3), (525000, 1)])
+def test_gradients_over_several_slabs(n, layers):
+    """Weight gradients are sums over chunks of rows, each staged in slabs of 32:
+    two slabs with a last chunk of one row, three with a ragged end, chunks of
+    288 rows (and of 69 for the edge layers), and the largest, 2,048 rows.
+    Within 1e-4 of each gradient's largest value, as at the tiles' edges; a
+    slab left out or taken twice would be off by about 1/sqrt(chunks) of it."""
+    net, p, X, T, nbr = problem(n, layers=layers, seed=2)
+    loss, g = net.gradient()
+    lr, gr = mpnn.backward({k: v.astype(np.float64) for k, v in p.items()}, X.astype(np.float64), nbr,
+                           T.astype(np.float64))
+    assert loss == pytest.approx(lr, rel=1e-5)
+    for k in gr:
+        assert np.max(np.abs(g[k] - gr[k])) <= 1e-4 * np.max(np.abs(gr[k])), k
+
+
+@pytest.mark.parametrize("big", [0, 1])
+def test_weight_gradients_of_values_that_do_not_split(big):
+    """Two rows, each the other's neighbour, only the first with a loss: A's
+    gradient holds the row's own feature times dz, B's the neighbour's.  One
+    of the two features is past the splitting range."""
+    net, p, X, T, _ = problem(2, layers=1)
+    for k in p:
+        p[k][...] = 0
+    p["W0"][0, 5] = 1.0
+    p["c"][0, 9] = 1.0
+    p["Wo"][9, 0] = 2.0 ** -10
+    X[...] = 0
+    X[:, 0] = (3.4e38, 3.0) if big == 0 else (3.0, 3.4e38)
+    T[...] = 0
+    T[1, 0] = 2.0 ** -10  # what the second row gives: z = 1, y = 2^-10
+    net.set_params(p)
+    net.set_data(X, T)
+    g = net.gradient()[1]
+    dz = np.float32(g["c"][0, 9])
+    assert dz > 0 and g["c"][0].astype(bool).sum() == 1
+    for name, x in (("A", X[0, 0]), ("B", X[1, 0])):
+        want = np.zeros((128, 128), np.float32)
+        want[5, 9] = x * dz
+        assert np.allclose(g[name][0], want, rtol=2.0 ** -23, atol=0), name

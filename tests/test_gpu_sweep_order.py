@@ -1,7 +1,7 @@
 """Storage in sweep-level order and the dataflow sweeps over it, at the shapes
 where an order or a chunk can go wrong: one cell, levels of exactly 64 and of
 65 cells, one-cell levels, a random numbering (many short levels), a colour
-numbering (two levels of half the mesh, six lower neighbours), a wide one past
+numbering (two levels of half the mesh, six lower neighbours), wide ones past
 the quad form's limit of cells per level, a batch.  Every comparison is bitwise:
 the order only moves where a cell's data live."""
 import numpy as np
@@ -177,3 +177,76 @@ def test_graphs_with_one_direction_in_dataflow_form(wide_first):
         for k in ("q", "res", "dq", "delta_flux"):
             assert np.array_equal(a.get_field(k), b.get_field(k)), (n, k)
     assert a.launch_counts()[0] >= 6
+
+
+def wide_levels(slots, count):
+    """One mesh of `count` disconnected blocks, so that a level holds a level of
+    every block: 27 cells in 7 levels with at most three swept neighbours, or 36
+    cells in 6 levels with four (two i-planes exchanged, so that one has both
+    its i-neighbours before it and the other both after it)."""
+    if slots == 3:
+        part = pa.Mesh.bump_hex(3, 3, 3)
+    else:
+        i, jk = np.arange(36) % 4, np.arange(36) // 4
+        part = pa.Mesh.bump_hex(4, 3, 3).renumbered("perm", 4 * jk + np.array([0, 2, 1, 3])[i])
+    c = pa.Mesh.concat([part] * count).connectivity()
+    return pa.Mesh.from_arrays(c["x"], c["y"], c["z"], c["face_node_ptr"], c["face_nodes"], c["left"], c["right"],
+                               c["n_bface"], c["bc_type"], c["cell_node_ptr"], c["cell_nodes"])
+
+
+WIDE = {3: 4667, 4: 3001}  # blocks: just past 18,000 cells per level
+INVISCID, TURBULENT = dict(viscous=0, reynolds=0.0), dict(viscous=3, cfl_start=0.5, cfl_end=0.5)
+
+
+@pytest.mark.parametrize("slots,count,form,over", [
+    (3, WIDE[3], 0, INVISCID), (3, WIDE[3], 0, dict(precision=1)), (3, WIDE[3], 0, TURBULENT), (3, WIDE[3], 2, {}),
+    (3, WIDE[3], 3, TURBULENT), (4, WIDE[4], 0, INVISCID), (4, WIDE[4], 0, dict(precision=1)),
+    (4, WIDE[4], 0, TURBULENT), (4, WIDE[4], 2, TURBULENT), (4, WIDE[4], 3, {}),
+    (4, 3000, 0, TURBULENT),  # at the limit: four lanes per cell
+])
+def test_wide_levels_with_64_cells_per_wavefront(slots, count, form, over):
+    mesh = wide_levels(slots, count)
+    fwd, bwd = pa.Solver(mesh, pa.default_params()).sweep_levels()
+    assert fwd == bwd == {3: 7, 4: 6}[slots]
+    assert (mesh.n_cell > 18000 * fwd) == (count != 3000)
+    a, b = run(mesh, 4, sweep_form=form, **over), run(mesh, 4, sweep_form=1, **over)
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
+
+
+def test_wide_levels_of_a_batch():
+    """The same blocks as cases with their own Mach numbers."""
+    mesh = pa.Mesh.concat([pa.Mesh.bump_hex(3, 3, 3)] * WIDE[3])
+    out = []
+    for form in (0, 1):
+        s = pa.Solver(mesh, [pa.default_params(mach=0.3 + 0.0001 * k, cfl_start=5.0, cfl_end=5.0, precision=1,
+                                               sweep_form=form) for k in range(WIDE[3])])
+        s.init_freestream()
+        out.append((s.iterate(1, 10), s.get_state(), s.get_field("dq")))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("bits", [0xFFFFFFFFFFFFFFFF, 0x7FF8000000000000])
+@pytest.mark.parametrize("name", ["levels_of_65", "two_wide_levels"])  # 16 and 64 cells per wavefront
+def test_not_a_number_in_the_state_is_no_mark(name, bits):
+    """A NaN of the caller's whose bits are those of the mark of an increment that
+    is not there yet: sweeps must not wait for it (the wait bound would be
+    reported), and spread it as the level form does."""
+    mesh = shapes()[name]()
+    q = perturbed_state(mesh.n_total, mesh.n_cell, FREE, 5, amp=0.01)
+    q[:, mesh.n_cell // 3] = np.array([bits], np.uint64).view(np.float64)[0]
+    out = []
+    for form in (0, 1):
+        s = pa.Solver(mesh, pa.default_params(mach=0.5, cfl_start=2.0, cfl_end=2.0, viscous=1, reynolds=5e4,
+                                              sweep_form=form))
+        s.init_freestream()
+        s.set_state(q)
+        s.residual()
+        s.spectrum_radius()
+        s.time_step(1)
+        s.lusgs()
+        out.append([s.get_field(k) for k in ("dq", "delta_flux", "q")])
+    assert np.isnan(out[0][0]).any()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b, equal_nan=True)
