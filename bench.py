@@ -256,24 +256,25 @@ def time_to_drop(mesh, pover, drop, max_steps, chunk=256, stall=2048):
 
 
 COPY_BYTES = 2 * 1024**3  # the calibration copy: 1 GiB read and 1 GiB written per launch
+TRAFFIC_STEPS = 4         # eager steps of a counter pass
 
 
 def traffic_child(cfg):
-    """The workload of a counter pass: two warm-up and two eager steps,
-    then the calibration copy."""
+    """The workload of a counter pass: TRAFFIC_STEPS eager steps, then the
+    calibration copy."""
     mesh = build_mesh(cfg["mesh"])
     s = pa.Solver(mesh, pa.default_params(**cfg["params"]))
     s.set_launch_mode("eager")
     s.init_freestream()
-    s.iterate(1, 4, history=False)
+    s.iterate(1, TRAFFIC_STEPS, history=False)
     s.synchronize()
     s.close()
     pa.hbm_copy_gbps(0, COPY_BYTES, 2)
 
 
 def _counter_means(out_dir):
-    """Mean counter value per dispatch, by (kernel, counter), from a
-    rocprofv3 csv counter collection."""
+    """(mean counter value per dispatch, dispatches), by (kernel, counter),
+    from a rocprofv3 csv counter collection."""
     import csv
     import glob
     sums = {}
@@ -287,7 +288,7 @@ def _counter_means(out_dir):
                 v = sums.setdefault(key, [0.0, 0])
                 v[0] += float(row["Counter_Value"])
                 v[1] += 1
-    return {k: v[0] / v[1] for k, v in sums.items() if v[1]}
+    return {k: (v[0] / v[1], v[1]) for k, v in sums.items() if v[1]}
 
 
 def measure_traffic(config, prefixes, counters=(("FETCH_SIZE",), ("WRITE_SIZE",)), timeout=240):
@@ -295,15 +296,15 @@ def measure_traffic(config, prefixes, counters=(("FETCH_SIZE",), ("WRITE_SIZE",)
     `prefixes`, measured in this run: one rocprofv3 counter pass per counter
     set over a short child run of the same workload, each counter scaled by
     what it reads for the copy kernel of known size in the same pass (1 GiB
-    read, 1 GiB written).  Returns {kernel: bytes} and the scale factors, or
-    None if the profiler is not available."""
+    read, 1 GiB written).  Returns {kernel: bytes}, each kernel's dispatches
+    per step and the scale factors, or None if the profiler is not available."""
     import shutil
     import subprocess
     import tempfile
     exe = shutil.which("rocprofv3")
     if not exe:
         return None
-    per_kernel, factors = {}, {}
+    per_kernel, per_step, factors = {}, {}, {}
     work = tempfile.mkdtemp(prefix="phl_pmc_", dir="/tmp")
     env = dict(os.environ, TMPDIR="/tmp")
     try:
@@ -322,17 +323,25 @@ def measure_traffic(config, prefixes, counters=(("FETCH_SIZE",), ("WRITE_SIZE",)
                 if not copy:
                     return None
                 # a copy launch reads and writes COPY_BYTES / 2 each
-                factor = (COPY_BYTES / 2) / (copy * 1024.0)
+                factor = (COPY_BYTES / 2) / (copy[0] * 1024.0)
                 factors[cname] = factor
-                for (kname, c2), v in means.items():
+                for (kname, c2), (v, n) in means.items():
                     if c2 == cname and any(kname.startswith(p) for p in prefixes):
                         per_kernel.setdefault(kname, {})[cname] = v * 1024.0 * factor
+                        per_step[kname] = n / TRAFFIC_STEPS
     except (OSError, subprocess.TimeoutExpired) as e:
         print(f"[bench] counter pass not run: {e}", file=sys.stderr, flush=True)
         return None
     finally:
         shutil.rmtree(work, ignore_errors=True)
-    return dict(kernels=per_kernel, factors=factors)
+    return dict(kernels=per_kernel, per_step=per_step, factors=factors)
+
+
+def step_traffic(tr, prefixes):
+    """Bytes per step of the kernels of measure_traffic whose names start with
+    one of `prefixes` (the two sweeps of a step may be one kernel or two)."""
+    ks = [k for k in tr["kernels"] if any(k.startswith(p) for p in prefixes)]
+    return sum(tr["per_step"][k] * sum(tr["kernels"][k].values()) for k in ks) if ks else None
 
 
 def wing_time_to_drop(mesh, pover, drop, max_steps, weights, chunk=256, stall=1024):
@@ -565,7 +574,7 @@ def mpnn_throughput(n_cases, dims, steps, layers=6):
     net.close()
     peak = 157.3e12
     out = dict(workload=f"{n_cases} bump-channel hex cases of {dims[0]}x{dims[1]}x{dims[2]} as one graph, "
-                        f"{layers} layers, width 128, FP32 (MFMA 32x32x2 f32), synthetic features",
+                        f"{layers} layers, width 128, FP32 (products of BF16 pieces, MFMA 32x32x16), synthetic features",
                cells=n, steps=steps)
     for key, t, train, pk in (("forward", t_fwd, False, peak), ("train_step", t_train, True, peak),
                               ("forward_bf16", t_fwd16, False, 2.5e15)):
@@ -613,7 +622,7 @@ def main():
     ap.add_argument("--sweep-form", default=None, choices=["dataflow", "levels", "ticket", "xcd"],
                     help="LU-SGS sweep form (default: the library's, dataflow in launch order)")
     ap.add_argument("--storage-order", default=None, choices=["locality", "mesh"],
-                    help="device storage order of the cells (default: the library's, locality)")
+                    help="device storage order of the cells (default: the library's, by sweep level)")
     ap.add_argument("--converge", type=float, default=None, metavar="DROP",
                     help="also time the FP64 and mixed-then-FP64 forms to this residual drop from freestream")
     ap.add_argument("--max-steps", type=int, default=20000, help="iteration cap of --converge")
@@ -721,11 +730,8 @@ def main():
     if not args.no_traffic and not cfg.get("batch"):
         tr = measure_traffic(args.config, ("k_sweep_flow", "k_face_flux", "k_cell_gather"))
         if tr:
-            def total(prefixes):
-                ks = [k for k in tr["kernels"] if any(k.startswith(p) for p in prefixes)]
-                return sum(sum(tr["kernels"][k].values()) for k in ks) if ks else None
-            roof_sweep["traffic"] = total(("k_sweep_flow",))
-            roof_face["traffic"] = total(("k_face_flux", "k_cell_gather"))
+            roof_sweep["traffic"] = step_traffic(tr, ("k_sweep_flow",))
+            roof_face["traffic"] = step_traffic(tr, ("k_face_flux", "k_cell_gather"))
             roof["traffic_per_kernel"] = {k: {c: round(v) for c, v in d.items()} for k, d in tr["kernels"].items()}
             roof["traffic_calibration"] = {c: round(f, 4) for c, f in tr["factors"].items()}
 
