@@ -76,12 +76,13 @@ typedef struct phl_params {
     int face_loop;          /* 0 (default): face kernel + cell gather, face values through HBM; 1:
                              * tile-fused (a workgroup evaluates the faces of its cells into LDS and sums
                              * them; faces between tiles are evaluated twice).  Identical results; the
-                             * tile form measured slower on the hybrid meshes (1M-cell hybrid bump:
-                             * 0.39 vs 0.32 ms). */
+                             * tile form measured slower (1M-cell hybrid bump: 0.40 vs 0.30 ms).  The
+                             * split form runs where a tile's face values exceed 64 KB of LDS. */
     int sweep_form;         /* LU-SGS sweeps (identical results: same arithmetic and summation order):
-                             * 0 (default) dataflow, one launch per direction: chunks of 64 cells of
-                             * the level order, each wavefront polling its swept neighbours' increments
-                             * until they are there, chunks taken in launch order;
+                             * 0 (default) dataflow, one launch per direction: chunks of the level
+                             * order, one per wavefront (16 cells of four lanes each up to a mean of
+                             * 18,000 cells per level, 64 cells beyond), each polling its swept
+                             * neighbours' increments until they are there, in launch order;
                              * 1 one launch per dependency level;
                              * 2 dataflow with chunks taken from a ticket counter (independent of the
                              * workgroup dispatch order; slower on large meshes);

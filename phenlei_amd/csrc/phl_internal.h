@@ -244,7 +244,11 @@ struct SweepOrder {
 // 254k (1,100) 0.50 + 0.50 against 0.35 + 0.34, wing of 2.24M (6,200) 0.90 +
 // 1.04 against 0.81 + 0.83; batches with 10,300 per level 0.92 + 0.93 against
 // 0.74 + 0.82, with 19,300 1.20 + 1.24 against 1.14 + 1.31, with 29,300 1.53 +
-// 1.63 against 1.62 + 1.89.
+// 1.63 against 1.62 + 1.89.  Laminar hybrid batches with 9,200 per level 0.24 +
+// 0.27 against 0.21 + 0.25, with 15,400 0.30 + 0.34 against 0.28 + 0.37, with
+// 24,700 0.39 + 0.48 against 0.41 + 0.56 (FP64 and mixed alike); turbulent wing
+// blocks with 11,700 0.33 + 0.33 against 0.29 + 0.30, with 19,500 0.42 + 0.45
+// against 0.41 + 0.46.
 constexpr int kQuadLevel = 18000;  // cells per level up to which the quad form is built
 struct FlowOrder {
     int nChunks;        // 0: not built

@@ -2217,11 +2217,12 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_block_so(DevMesh M, Const
 // took 1.53 + 1.56 ms on the 2.24M-cell wing, 0.99 + 0.99 on the 1.01M-cell
 // hybrid channel, 0.60 + 0.63 on the 254k-cell and 0.23 + 0.27 on the 16k-cell
 // hex channel; marks take 0.90 + 1.04, 0.55 + 0.57, 0.50 + 0.50 and 0.20 +
-// 0.20 (64 cells per wavefront).  A flag published early as a hint, before polling the rows, was slower
-// than polling at once (wing 1.10 + 1.22).
+// 0.20 (64 cells per wavefront).  A flag published early as a hint, before
+// polling the rows, was slower than polling at once (wing 1.10 + 1.22).
 // Polling the rows pays only because they are few lines: storage follows the
-// level order (sweep_order), so the 64 neighbours of a slot lie in short runs
-// of rows, and the pair planes (kPlanes) keep a run contiguous.
+// level order (sweep_storage_order on the host), so the neighbours that a
+// chunk's cells have in one slot lie in short runs of rows, and the pair planes
+// (kPlanes) keep a run contiguous.
 // ctl: [0] ticket (sweep_form 2), [2] waves that gave up, [3] the wait bound
 // in ticks of the 100 MHz wall clock (set by the host; 20,000,000 = 0.2 s by
 // default).

@@ -149,7 +149,7 @@ __device__ __forceinline__ unsigned not_finite(const f32x16 (&acc)[2][2])
 // 16 k take 192 cycles against 512.  Its error against 64 bits is no larger:
 // network output 2.5e-7 against 2.9e-7 (200,704 rows), gradients (with
 // k_wgrad_part) 4.7e-8 against 2.4e-7 at 315 rows and as under kTerms at
-// 123,240.  A hidden layer of 200,704 rows takes 131 us instead of 262 (66 us
+// 123,240.  A hidden layer of 200,704 rows takes 134 us instead of 262 (66 us
 // are the bytes alone), bound by the latency of a workgroup's eight chunks at
 // two workgroups per CU.  NP 1 (inference) is bound by its 1,536 bytes of
 // activations per row: 621,818 rows in 224 us instead of 351, 4.3 TB/s.

@@ -420,12 +420,12 @@ def test_tile_fused_face_loop_runs(kind, viscous, storage):
                                                  ("hybrid", 0, 2), ("wing", 1, 2), ("hex", 0, 3), ("hybrid", 1, 3),
                                                  ("wing", 0, 3)])
 def test_dataflow_sweep_equals_level_sweep(kind, precision, form):
-    """The dataflow sweeps (one launch per direction, per-chunk flags; chunks
-    in launch order, form 0, ticket order, form 2, or split over the XCDs,
-    form 3) and the level-by-level
-    launches (form 1) apply the same arithmetic in the same order: states,
-    residual histories and dq are bitwise equal, over several calls (the
-    flags carry a new epoch each sweep) and in both launch modes."""
+    """The dataflow sweeps (one launch per direction, waiting on marked
+    increments; chunks in launch order, form 0, ticket order, form 2, or split
+    over the XCDs, form 3) and the level-by-level launches (form 1) apply the
+    same arithmetic in the same order: states, residual histories and dq are
+    bitwise equal, over several calls (each sweep marks the buffer of the next)
+    and in both launch modes."""
     if kind == "hex":
         m = pa.Mesh.bump_hex(48, 16, 6, 0.08)
     elif kind == "wing":

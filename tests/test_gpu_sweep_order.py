@@ -59,14 +59,12 @@ def test_dataflow_sweep_at_chunk_edges_equals_level_form(name, form):
         assert np.array_equal(a[k], b[k]), (name, k)
 
 
-@pytest.mark.parametrize("over", [dict(), dict(viscous=3, cfl_start=0.5, cfl_end=0.5), dict(n_lusgs_sweeps=3)],
-                         ids=["laminar", "turbulent", "three_pairs"])
-@pytest.mark.parametrize("name", sorted(shapes()))
+@pytest.mark.parametrize("name,over", [(n, o) for n in sorted(shapes()) for o in (
+    {}, dict(viscous=3, cfl_start=0.5, cfl_end=0.5), dict(n_lusgs_sweeps=3)) if n != "batch" or not o])
 def test_level_form_in_mesh_order(name, over):
-    """Increments as rows of one line each instead of planes."""
+    """Increments as rows of one line each instead of planes (a batch is laminar,
+    with one sweep pair)."""
     mesh = shapes()[name]()
-    if mesh.n_cases > 1 and over:
-        pytest.skip("batched contexts are laminar or inviscid, with one sweep pair")
     a, b = run(mesh, 4, sweep_form=1, storage_order=1, **over), run(mesh, 4, **over)
     for k in a:
         assert np.array_equal(a[k], b[k]), (name, k)
