@@ -1534,10 +1534,23 @@ static phl_status clear_gave_up(phl_ctx *c)
     return PHL_OK;
 }
 
+static void join_turb(phl_ctx *c);
+
+// A turbulence relaxation that a failed phl_iterate left pending belongs to
+// the state that failed: its sweeps, if they run on the side stream, end before
+// the new state's fields are written, and if they wait for the next step they
+// are dropped.
+static void drop_pending(phl_ctx *c)
+{
+    join_turb(c);
+    c->saDeferred = false;
+}
+
 phl_status phl_set_state(phl_ctx *c, const double *q)
 {
     if (!c || !q) return fail(PHL_ERR_ARG, "null argument");
     HIPTRY(hipSetDevice(c->device));
+    drop_pending(c);
     ++c->stateVersion;
     c->tFresh = true;
     TRY(upload_cells(c, c->f.q, 5, c->m.nTotal, q));
@@ -1680,6 +1693,7 @@ phl_status phl_init_freestream(phl_ctx *c)
 {
     if (!c) return fail(PHL_ERR_ARG, "null argument");
     HIPTRY(hipSetDevice(c->device));
+    drop_pending(c);
     c->tFresh = true;
     const int nT = c->m.nTotal, nC = c->m.nCell;
     std::vector<double> h((size_t)5 * nT);

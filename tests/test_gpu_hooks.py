@@ -284,3 +284,30 @@ def test_context_recovers_when_another_error_hides_that_a_sweep_gave_up(form):
     ref.init_freestream()
     assert np.array_equal(s.iterate(1, 12), ref.iterate(1, 12))
     assert np.array_equal(s.get_state(), ref.get_state())
+
+
+@pytest.mark.parametrize("form,mode", [(0, "graph"), (0, "eager"), (1, "graph"), (1, "eager_overlap")])
+def test_turbulent_context_recovers_from_a_numeric_error(form, mode):
+    """phl_iterate stops on a residual that is not finite with a turbulence
+    relaxation still pending: it belongs to the state that failed, so a new
+    state (with its nu~ and eddy viscosity) starts without it."""
+    m = pa.Mesh.swept_wing(12, 6, 5, 1e-3, 3)
+    p = pa.default_params(mach=0.5, viscous=3, reynolds=1e5, cfl_start=0.5, cfl_end=0.5, sweep_form=form)
+    s, ref = pa.Solver(m, p), pa.Solver(m, p)
+    for c in (s, ref):
+        c.set_launch_mode(mode)
+        c.init_freestream()
+    q, nut, vist = ref.get_state(), ref.get_field("nut"), ref.get_field("vist")
+    bad = q.copy()
+    bad[:, m.n_cell // 2] = np.nan
+    s.set_state(bad)
+    with pytest.raises(pa.PhlError) as e:
+        s.iterate(1, 20)
+    assert e.value.status == pa.PHL_ERR_NUMERIC
+    for c in (s, ref):
+        c.set_state(q)
+        c.set_field("nut", nut)
+        c.set_field("vist", vist)
+    assert np.array_equal(s.iterate(1, 20), ref.iterate(1, 20))
+    for k in ("q", "nut"):
+        assert np.array_equal(s.get_field(k), ref.get_field(k)), k
